@@ -1152,105 +1152,127 @@ void merkle_lifted_leaves(const LeafSrc& L, uint32_t* hashes, hipStream_t s) {
 }
 
 // ------------------------------------------------------------- decommitment
-// One 64-lane workgroup per (tree, query, role): role 0 opens the query leaf,
-// role 1 its partner (the sibling, or the next row). Each re-hashes the
-// 2^lo-leaf group that holds its leaf, takes the path below level `lo` from
-// it and the rest from the stored levels, and writes its values and auth
-// path into the proof (src/bin/stark_cli.rs:1061-1089 layout: n, values,
-// partner values, paths, partner paths).
+// One wavefront opens two queries of a tree: 16 lanes per (query, role),
+// role 0 the query leaf, role 1 its partner (the sibling, or the next row).
+// The 16 lanes re-hash the 2^lo-leaf group (lo <= 4) that holds their leaf,
+// take the path below level `lo` from it and the rest from the stored
+// levels, and write values and auth path into the proof
+// (src/bin/stark_cli.rs:1061-1089 layout: n, values, partner values, paths,
+// partner paths).
+//
+// Bound by the instructions of the re-hash, a chain of lo compressions per
+// opening: with a wavefront per opening only 16 of its 64 lanes hashed, and
+// the four wavefronts a SIMD got of a 2^24 proof's 4,000 took turns. Packing
+// four openings leaves about one wavefront per SIMD; its levels of at most
+// 16 nodes (from the second up) are hashed by quads. Paths are copied by
+// lanes that each move one word of eight, so a node is one 32-byte run
+// (before: a lane per node, eight strided words). 80 queries: Fibonacci
+// log_n = 10 26.7 -> 9.9 us, log_n = 16 35.1 -> 11.6 us, 34 columns at
+// log_n = 17 37.9 -> 13.2 us.
 __device__ __forceinline__ uint32_t decom_width(const DecomDesc& d) {
   return (d.kind == DECOM_COLS || d.kind == DECOM_LIFTED) ? d.n_cols : 4u;
 }
-__device__ __forceinline__ void decom_value(const DecomDesc& d, uint64_t i, uint32_t w[16]) {
-  if (d.kind == DECOM_COLS) {
-    for (uint32_t c = 0; c < d.n_cols; c++) w[c] = d.col[c][i];
-  } else if (d.kind == DECOM_SOA4) {
-    for (int c = 0; c < 4; c++) w[c] = d.col[c][i];
-  } else {
+// The words of leaf i of a tree whose leaves are at most 16 words (the rest 0).
+__device__ __forceinline__ void decom_value(const DecomDesc& d, uint64_t i, uint32_t (&w)[16]) {
+#pragma unroll
+  for (uint32_t c = 0; c < 16; c++) w[c] = 0;
+  if (d.kind == DECOM_QUOTIENT) {
     const uint64_t mask = (1ull << d.log_n) - 1;
     const uint32_t* ev = d.col[0];
     uint32_t c = m31_sub(ev[(i + 2) & mask], m31_add(ev[(i + 1) & mask], ev[i]));
     qm31 q = qm_scale(ldq(d.alpha), c);
+#pragma unroll
     for (int k = 0; k < 4; k++) w[k] = q.v[k];
+  } else {
+    const uint32_t n = decom_width(d);
+#pragma unroll
+    for (uint32_t c = 0; c < 16; c++)
+      if (c < n) w[c] = d.col[c][i];
   }
 }
 
+static constexpr uint32_t DEC_GROUP = 16;  // lanes (and leaves at most) per opening
+
 __global__ __launch_bounds__(64) void k_decommit(const DecomDesc* descs, const uint32_t* queries, uint32_t nq,
                                                  uint32_t* proof) {
-  __shared__ uint32_t nodes[32 * 8];  // level v of the group at node offset 32 - 2^(lo - v + 1)
-  const uint32_t role = blockIdx.x & 1, tq = blockIdx.x >> 1;
-  const uint32_t tree = tq / nq, q = tq % nq;
-  const DecomDesc& d = descs[tree];
-  const uint32_t lane = threadIdx.x;
+  // level v of an opening's group at node offset 32 - 2^(lo - v + 1)
+  __shared__ uint4 nodes4[4][32 * 2];
+  const DecomDesc& d = descs[blockIdx.y];
+  const uint32_t g = threadIdx.x / DEC_GROUP, lane = threadIdx.x % DEC_GROUP;
+  const uint32_t role = g & 1, q = 2 * blockIdx.x + (g >> 1);
+  const bool on = q < nq;  // an odd last query leaves half the wavefront idle
   const uint32_t lo = d.lo, D = d.log_n, W = decom_width(d);
   const uint64_t mask = (1ull << D) - 1;
-  const uint64_t qidx = (uint64_t)queries[q] >> d.shift;
+  const uint64_t qidx = on ? (uint64_t)queries[q] >> d.shift : 0;
   const uint64_t idx = role == 0 ? qidx : (d.pair == PAIR_NEXT ? (qidx + 1) & mask : qidx ^ 1);
   const uint64_t first = (idx >> lo) << lo;
-  // level v occupies nodes [base(v), base(v) + 2^(lo-v)), base(v) = 32 - 2^(lo-v+1)
+  const uint64_t pair_words = ((uint64_t)role * nq + q) * W;
+  uint32_t* values = proof + d.proof_word + 1 + pair_words;
   if (lane < (1u << lo)) {
     uint32_t h[8];
     if (d.kind == DECOM_LIFTED) {
       lifted_leaf_cols(d.lift, d.n_cols, D, first + lane, h);
     } else {
       uint32_t w[16];
-      for (int k = 0; k < 16; k++) w[k] = 0;
       decom_value(d, first + lane, w);
       b2_hash_words(w, W, h);
+      if (on && first + lane == idx) {
+#pragma unroll
+        for (uint32_t k = 0; k < 16; k++)
+          if (k < W) values[k] = w[k];
+      }
     }
-    for (int k = 0; k < 8; k++) nodes[8 * (32 - (2u << lo) + lane) + k] = h[k];
+    lds_put(nodes4[g], 32 - (2u << lo) + lane, h);
   }
   __syncthreads();
   for (uint32_t v = 1; v < lo; v++) {
     const uint32_t cnt = 1u << (lo - v);
     const uint32_t src = 32 - (4u << (lo - v)), dst = 32 - (2u << (lo - v));
-    if (lane < cnt) {
-      uint32_t l[8], r[8], h[8];
-      for (int k = 0; k < 8; k++) {
-        l[k] = nodes[8 * (src + 2 * lane) + k];
-        r[k] = nodes[8 * (src + 2 * lane + 1) + k];
+    if (4 * cnt <= DEC_GROUP) {
+      const uint32_t nid = lane >> 2, quad = lane & 3;
+      if (nid < cnt) {
+        const uint32_t* in = reinterpret_cast<const uint32_t*>(nodes4[g]) + 8 * (src + 2 * nid);
+        uint32_t m[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) m[k] = in[k];
+        uint32_t h_lo, h_hi;
+        b2_node_x4(m, quad, h_lo, h_hi);
+        uint32_t* out = reinterpret_cast<uint32_t*>(nodes4[g]) + 8 * (dst + nid);
+        out[quad] = h_lo;
+        out[4 + quad] = h_hi;
       }
+    } else if (lane < cnt) {
+      uint32_t l[8], r[8], h[8];
+      lds_get(nodes4[g], src + 2 * lane, l);
+      lds_get(nodes4[g], src + 2 * lane + 1, r);
       b2_hash_node(l, r, h);
-      for (int k = 0; k < 8; k++) nodes[8 * (dst + lane) + k] = h[k];
+      lds_put(nodes4[g], dst + lane, h);
     }
     __syncthreads();
   }
-  const uint64_t base = d.proof_word;
-  const uint64_t pbase = base + 1 + 2ull * nq * W;
-  const uint64_t plen = 1 + 8ull * D;
-  uint32_t* path = proof + pbase + ((uint64_t)role * nq + q) * plen;
-  if (d.kind == DECOM_LIFTED) {  // the opened row: every column at its lifted row
-    for (uint32_t c = lane; c < W; c += 64)
-      proof[base + 1 + ((uint64_t)role * nq + q) * W + c] = d.lift[c].p[lifted_row(idx, D, d.lift[c].log_n)];
-    if (lane == 0) {
-      if (q == 0 && role == 0) proof[base] = nq;
-      path[0] = D;
-    }
-  } else if (lane == 0) {
-    uint32_t w[16];
-    if (q == 0 && role == 0) proof[base] = nq;
-    decom_value(d, idx, w);
-    for (uint32_t k = 0; k < W; k++) proof[base + 1 + ((uint64_t)role * nq + q) * W + k] = w[k];
+  if (!on) return;
+  if (d.kind == DECOM_LIFTED)  // the opened row: every column at its lifted row
+    for (uint32_t c = lane; c < W; c += DEC_GROUP) values[c] = d.lift[c].p[lifted_row(idx, D, d.lift[c].log_n)];
+  uint32_t* path = proof + d.proof_word + 1 + 2ull * nq * W + ((uint64_t)role * nq + q) * (1 + 8ull * D);
+  if (lane == 0) {
+    if (q == 0 && role == 0) proof[d.proof_word] = nq;
     path[0] = D;
   }
-  if (lane < D) {
-    const uint32_t v = lane;
-    const uint32_t* sib;
-    if (v < lo) {
-      const uint32_t lvl_base = 32 - (2u << (lo - v));
-      sib = &nodes[8 * (lvl_base + (uint32_t)(((idx >> v) ^ 1) - (first >> v)))];
-    } else {
-      sib = d.tree + d.off[v] + 8 * ((idx >> v) ^ 1);
-    }
-    for (int k = 0; k < 8; k++) path[1 + 8 * v + k] = sib[k];
+  const uint32_t* low = reinterpret_cast<const uint32_t*>(nodes4[g]);
+  for (uint32_t e = lane; e < 8 * D; e += DEC_GROUP) {
+    const uint32_t v = e >> 3, k = e & 7;
+    uint32_t x;
+    if (v < lo) x = low[8 * (32 - (2u << (lo - v)) + (uint32_t)(((idx >> v) ^ 1) - (first >> v))) + k];
+    else x = d.tree[d.off[v] + 8 * ((idx >> v) ^ 1) + k];
+    path[1 + e] = x;
   }
 }
 
 void decommit(const DecomDesc* d_descs, uint32_t n_trees, const uint32_t* d_queries, uint32_t nq, uint32_t* proof,
               hipStream_t s) {
   if (n_trees == 0 || nq == 0) return;
-  require((uint64_t)n_trees * nq * 2 < (1ull << 31), "decommit: too many openings");
-  hipLaunchKernelGGL(k_decommit, dim3(2 * n_trees * nq), dim3(64), 0, s, d_descs, d_queries, nq, proof);
+  require(n_trees <= 65535 && (uint64_t)n_trees * nq * 2 < (1ull << 31), "decommit: too many openings");
+  hipLaunchKernelGGL(k_decommit, dim3((nq + 1) / 2, n_trees), dim3(64), 0, s, d_descs, d_queries, nq, proof);
   VX_HIP(hipGetLastError());
 }
 
