@@ -608,12 +608,11 @@ __device__ __forceinline__ void finish_root_q0(const RootHook& h, const uint32_t
 // Merges `nthr` nodes held one per lane in `buf[0]` up to one node, storing
 // each produced level (lvl0+1 ...) at global index base_idx(level) + lane.
 // Returns the top node in lane 0's `node`.
-// With QUAD, levels with at most CAP / 4 nodes hash each node with the four
-// lanes of a quad (b2_node_x4): those levels are a dependent chain with most
-// lanes idle, so halving the instructions per compression halves their
-// latency. (The throughput instances do without: the quad path raises their
-// VGPR count.) Lanes 0..3 return the top node.
-template <uint32_t CAP, bool QUAD>
+// Levels with at most CAP / 4 nodes hash each node with the four lanes of a
+// quad (b2_node_x4): those levels are a dependent chain with most lanes idle,
+// so halving the instructions per compression halves their latency. Lanes
+// 0..3 return the top node.
+template <uint32_t CAP>
 __device__ __forceinline__ void lds_merge(uint4 (*buf)[2 * CAP], uint32_t nthr, uint32_t lvl0,
                                           const TreeLevels& T, uint64_t group, uint32_t group_log,
                                           uint32_t store_lo, uint32_t node[8]) {
@@ -622,7 +621,7 @@ __device__ __forceinline__ void lds_merge(uint4 (*buf)[2 * CAP], uint32_t nthr, 
   uint32_t cnt = nthr;
   for (uint32_t lvl = lvl0 + 1; cnt > 1; lvl++) {
     cnt >>= 1;
-    if (QUAD && 4 * cnt <= CAP) {
+    if (4 * cnt <= CAP) {
       const uint32_t nid = tid >> 2, q = tid & 3;
       if (nid < cnt) {
         const uint32_t* src = reinterpret_cast<const uint32_t*>(buf[cur]) + 16 * nid;
@@ -655,13 +654,68 @@ __device__ __forceinline__ void lds_merge(uint4 (*buf)[2 * CAP], uint32_t nthr, 
   if (tid < 4) lds_get(buf[cur], 0, node);
 }
 
+// The same merge for the throughput instances: in place on messages
+// QUAD_STRIDE words apart (child c of a level is half of message c >> 1), quad
+// levels by b2_hash_x4_lds. A tile of 1,024 leaves issues about 35,000
+// wavefront instructions, 4,800 of them in these levels with the register
+// form and 3,800 here; Fibonacci log_n = 24 proof 11.93 -> 11.65 ms.
+__host__ __device__ constexpr uint32_t lds_nodes(uint32_t n) { return n / 2 * QUAD_STRIDE; }  // words for n children
+__device__ __forceinline__ uint32_t* lds_node(uint32_t* s, uint32_t c) {
+  return s + QUAD_STRIDE * (c >> 1) + 8 * (c & 1);
+}
+__device__ __forceinline__ void lds_merge_in_place(uint32_t* s, uint32_t cnt, uint32_t lvl, const TreeLevels& T,
+                                                   uint64_t group, uint32_t group_log, uint32_t store_lo) {
+  const uint32_t tid = threadIdx.x, nid = tid >> 2, q = tid & 3;
+  const QuadOff o = quad_off(quad_row(q), 4 * QUAD_STRIDE * nid);
+  while (cnt > 1) {
+    cnt >>= 1;
+    lvl++;
+    // levels of at most 16 nodes are the first wavefront's: no barrier
+    const bool solo = cnt <= 16;
+    if (solo && tid >= 64) return;
+    const bool store = T.base && lvl >= store_lo;
+    uint32_t* g = store ? T.base + T.off[lvl] + 8 * (group << (group_log - lvl)) : nullptr;
+    if (4 * cnt <= SUB_THREADS) {
+      uint32_t lo = 0, hi = 0;
+      if (nid < cnt) b2_hash_x4_lds(s, o, 64u, q, lo, hi);
+      if (!solo) __syncthreads();  // every child read before any parent overwrites it
+      if (nid < cnt) {
+        uint32_t* dst = lds_node(s, nid);
+        dst[q] = lo;
+        dst[4 + q] = hi;
+        if (store) {
+          g[8 * nid + q] = lo;
+          g[8 * nid + 4 + q] = hi;
+        }
+      }
+    } else {
+      uint32_t node[8];
+      if (tid < cnt) {
+        uint32_t m[16];
+        const uint32_t* c = lds_node(s, 2 * tid);
+#pragma unroll
+        for (int k = 0; k < 4; k++) u4w(ld4(c + 4 * k), m + 4 * k);
+        b2_hash_node(m, m + 8, node);
+      }
+      __syncthreads();
+      if (tid < cnt) {
+        store_node(lds_node(s, tid), node);
+        if (store) store_node(g + 8 * tid, node);
+      }
+    }
+    if (solo) wave_lds_order();
+    else __syncthreads();
+  }
+}
+
 // ROOT instances (the whole tree in one workgroup) carry the transcript step;
 // the throughput instances do not, which keeps their VGPR count (and so their
 // occupancy) at what the hashing itself needs.
 template <uint32_t KIND, uint32_t NC, uint32_t LPT_LOG, bool ROOT>
 __global__ __launch_bounds__(SUB_THREADS) void k_subtree(LeafSrc L, TreeLevels T, uint32_t tile_log,
                                                          uint32_t store_lo, RootHook hook) {
-  __shared__ uint4 buf[2][2 * SUB_THREADS];
+  constexpr bool IN_PLACE = !ROOT && LPT_LOG >= 2;
+  __shared__ uint4 buf[IN_PLACE ? 1 : 2][IN_PLACE ? lds_nodes(SUB_THREADS) / 4 : 2 * SUB_THREADS];
   const uint32_t nthr = 1u << (tile_log - LPT_LOG);
   const uint32_t tid = threadIdx.x;
   const uint64_t tile = blockIdx.x;
@@ -685,12 +739,16 @@ __global__ __launch_bounds__(SUB_THREADS) void k_subtree(LeafSrc L, TreeLevels T
     const uint64_t first = (tile << tile_log) + ((uint64_t)tid << LPT_LOG);
     if constexpr (LPT_LOG == 0) lane_leaf<KIND, NC>(L, first, node);
     else lane_subtree<KIND, NC, LPT_LOG>(L, first, node);
-    lds_put(buf[0], tid, node);
+    if constexpr (IN_PLACE) store_node(lds_node(reinterpret_cast<uint32_t*>(buf), tid), node);
+    else lds_put(buf[0], tid, node);
     if (T.base && LPT_LOG >= store_lo)
       store_node(T.base + T.off[LPT_LOG] + 8 * ((tile << (tile_log - LPT_LOG)) + tid), node);
   }
   __syncthreads();
-  lds_merge<SUB_THREADS, ROOT || LPT_LOG <= 2>(buf, nthr, LPT_LOG, T, tile, tile_log, store_lo, node);
+  if constexpr (IN_PLACE)
+    lds_merge_in_place(reinterpret_cast<uint32_t*>(buf), nthr, LPT_LOG, T, tile, tile_log, store_lo);
+  else
+    lds_merge<SUB_THREADS>(buf, nthr, LPT_LOG, T, tile, tile_log, store_lo, node);
   if constexpr (ROOT) {
     if (tid < 4) finish_root_q0(hook, node, tid);
   }
@@ -734,7 +792,7 @@ __global__ __launch_bounds__(RED_THREADS) void k_tree_reduce(TreeLevels T, uint3
     store_node(T.base + T.off[from + 1] + 8 * ((wg << (nlev - 1)) + tid), node);
   }
   __syncthreads();
-  lds_merge<RED_THREADS, true>(buf, nthr, from + 1, T, wg, from + nlev, 0, node);
+  lds_merge<RED_THREADS>(buf, nthr, from + 1, T, wg, from + nlev, 0, node);
   if constexpr (ROOT) {
     if (tid < 4) finish_root_q0(hook, node, tid);
   }
@@ -1089,7 +1147,7 @@ __global__ __launch_bounds__(RTR_THREADS) void k_reduce_to_root(const uint32_t* 
   }
   __syncthreads();
   TreeLevels none{};
-  lds_merge<RTR_THREADS, true>(buf, nthr, 0, none, 0, 0, 0, node);
+  lds_merge<RTR_THREADS>(buf, nthr, 0, none, 0, 0, 0, node);
   if (tid == 0)
     for (int k = 0; k < 8; k++) root[k] = node[k];
 }
