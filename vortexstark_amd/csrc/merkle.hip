@@ -178,8 +178,6 @@ __device__ __forceinline__ void leaf_produce(const LeafSrc& L, uint64_t i, const
 // constraints and reduced once at the end. The constraint table and weights
 // are wave-uniform (scalar loads); the rows are one 16-byte load per column
 // use plus the wrapped row i + 4 of column b. Q is stored (SoA) for the fold.
-__device__ __forceinline__ uint64_t fold64(uint64_t x) { return (x & 0xFFFFFFFFull) + ((x >> 32) << 1); }
-
 __device__ __forceinline__ void d2_produce(const LeafSrc& L, uint64_t i, G4& g, bool store = true) {
   const uint32_t* ev = L.col[0];
   const uint64_t st = L.col_stride;
@@ -217,7 +215,7 @@ __device__ __forceinline__ void d2_produce(const LeafSrc& L, uint64_t i, G4& g, 
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) acc[j][c] = fold64(acc[j][c]);
+      for (int c = 0; c < 4; c++) acc[j][c] = m31_fold64(acc[j][c]);
   }
 #pragma unroll
   for (int j = 0; j < 4; j++)
@@ -359,7 +357,7 @@ __device__ __forceinline__ void lifted_rlc_produce(const LeafSrc& L, uint64_t i,
 #pragma unroll
       for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) acc[j][k] = fold64(acc[j][k]);
+        for (int k = 0; k < 4; k++) acc[j][k] = m31_fold64(acc[j][k]);
     }
   } else
   for (uint32_t c0 = 0; c0 < n; c0 += 4) {
@@ -388,7 +386,7 @@ __device__ __forceinline__ void lifted_rlc_produce(const LeafSrc& L, uint64_t i,
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int k = 0; k < 4; k++) acc[j][k] = fold64(acc[j][k]);
+      for (int k = 0; k < 4; k++) acc[j][k] = m31_fold64(acc[j][k]);
   }
 #pragma unroll
   for (int j = 0; j < 4; j++)

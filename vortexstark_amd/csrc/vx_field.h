@@ -96,11 +96,20 @@ VX_HD qm31 fri_fold_pair(qm31 f0, qm31 f1, qm31 alpha, uint32_t tw) {
   return qm_add(qm_add(f0, f1), qm_mul(alpha, qm_scale(qm_sub(f0, f1), tw)));
 }
 
-// x mod P of any 64-bit x: fold at bit 31 twice, then canonicalise.
+// lo + 2 hi of x = hi 2^32 + lo: congruent to x mod P (2^32 = 2), below
+// 3 * 2^32. On the device one v_mad_u64_u32: the factor is kept from the
+// compiler, which makes it a 64-bit shift, mask and add otherwise.
+VX_HD uint64_t m31_fold64(uint64_t x) {
+  uint32_t two = 2;
+#ifdef __HIP_DEVICE_COMPILE__
+  asm("" : "+s"(two));
+#endif
+  return (x >> 32) * (uint64_t)two + (uint32_t)x;
+}
+// x mod P of any 64-bit x: folded at bit 32, then at bit 31, then made canonical.
 VX_HD uint32_t m31_reduce64(uint64_t x) {
-  const uint64_t s = (x & P) + (x >> 31);               // < 2^34
-  const uint32_t r = (uint32_t)((s & P) + (s >> 31));  // < 2^31 + 8
-  return m31_canon(r);
+  const uint64_t s = m31_fold64(x);
+  return m31_canon(((uint32_t)s & P) + (uint32_t)(s >> 31));  // of a sum below 2^31 + 6
 }
 
 // Left multiplication by a fixed QM31 x as a 4x4 matrix over M31 (u^2 =
