@@ -214,250 +214,290 @@ const uint32_t* eval_at_point(const uint32_t* c, const uint32_t* factors, uint32
 }
 
 // ---------------------------------------------------------------------------
-// Many columns at one point (the OODS step evaluates every committed column
-// at z; cuda/batch_eval_at_point.cu:11-100 restricts this to n <= 64). A
-// column of 2^L coefficients uses the last L of the max_log_n factors, so
-// coefficient bit b of every column is folded by the same
-// F[b] = factors[max_log_n - 1 - b]. Columns are cut into chunks of 2^14
-// coefficients (shorter columns are one chunk, the words past their end
-// read as zero, which no factor can change), and one launch runs every
-// chunk of every column with the k_eval_big arithmetic (work list: each
-// workgroup binary-searches its column). Per column, the chunk sums are
-// then folded 256 at a time with F[14..], one launch per level for all
-// columns.
-struct EvalChunkJob {
-  const uint32_t* col;
-  uint32_t log_n;
-  uint32_t first_chunk;  // jobs sorted by first_chunk
+// Many columns at one or two points (the OODS step evaluates every committed
+// column at z and at z_next; cuda/batch_eval_at_point.cu:11-100 restricts
+// this to n <= 64). A column of 2^L coefficients uses the last L of the
+// max_log_n factors, so coefficient bit b of every column is folded by the
+// same F[b] = factors[max_log_n - 1 - b], and the weight of a coefficient is
+// a product over its index bits. Columns are cut into chunks of 2^14
+// coefficients (shorter columns are one chunk, the words past their end read
+// as zero); in a chunk lane t reads the 16 uint4 at t + 256 m, so index bits
+// 0-1 are the component r, 2-9 the lane, 10-13 m, and from 14 up the chunk:
+//   f(z) = sum_chunk G[chunk] sum_t L[t] sum_j E[j] c,  j = (r, m), 64 values.
+// The tables E, L and G are made once per call (k_eval_tables). A workgroup
+// takes some consecutive chunks of a column: per chunk each lane forms its
+// 64-term sums against E (wave-uniform scalars) and adds G[chunk] times them
+// to its own; L[t] and the sum over the lanes follow once at the end, and a
+// second launch adds the workgroups' sums.
+//
+// Bound by the read of the columns once the arithmetic is small: a term is
+// one multiply-add per component into a signed 64-bit sum (weights centred to
+// |w| < 2^30, coefficients shifted by 2^30, so eight products fit before a
+// fold; the shift's share of the sum is the constant C). The tree folds of
+// the lanes by QM31 products that this replaces were two thirds of the
+// kernel's instructions. 64 columns of 2^20 at two points (268 MB): 192 -> 51 us
+// (the read at a large copy's rate takes 52); the OODS step 338 -> 133 us.
+static constexpr uint32_t EV_TERMS = 64;      // coefficients per lane and chunk
+static constexpr uint32_t EV_MAX_WGS = 2048;  // of a call: chunks per workgroup grow beyond
+static constexpr uint32_t EV_ARG_COLS = 192;  // columns per launch (kernel arguments)
+
+struct EvalCols {
+  const uint32_t* col[EV_ARG_COLS];
+  uint32_t first[EV_ARG_COLS];  // workgroup of the column's first chunk, ascending from 0
+  uint8_t log_n[EV_ARG_COLS];
+  uint32_t n, cpw_log, wg_base;  // 2^cpw_log chunks per workgroup; wg_base: workgroups of earlier launches
 };
-struct EvalFoldJob {
-  uint32_t in;   // first QM31 of the group in the input level
-  uint32_t out;  // its QM31 in the output level
-  uint32_t n;    // sums in the group (a power of two, <= 256)
-  uint32_t fb;   // coefficient bit folded by the group's level 0
+// words of the tables of np points, G having 2^g_log entries
+struct EvalTables {
+  uint32_t np, g_log;
+  __host__ __device__ uint64_t e() const { return 0; }                              // [64][np] centred QM31
+  __host__ __device__ uint64_t c() const { return 4ull * EV_TERMS * np; }           // [np]
+  __host__ __device__ uint64_t l() const { return c() + 4ull * np; }                // [np][256]
+  __host__ __device__ uint64_t g() const { return l() + 4ull * EV_WG * np; }        // [np][2^g_log]
+  __host__ __device__ uint64_t words() const { return g() + (4ull * np << g_log); }
 };
 
 __device__ __forceinline__ qm31 factor_or_one(const uint32_t* factors, uint32_t max_log_n, uint32_t b) {
   return b < max_log_n ? ld_factor(factors, max_log_n, b) : qm31{{1u, 0u, 0u, 0u}};
 }
 
-// table: E[16] over bits {0,1,10,11}, D[4] over {12,13}, F[2..9] at 20..27
-__global__ void k_eval_batch_setup(const uint32_t* factors, uint32_t max_log_n, uint32_t* table) {
-  const uint32_t q = threadIdx.x;
-  qm31 b{{1u, 0u, 0u, 0u}};
-  if (q < 16) {
-    const uint32_t bits[4] = {0, 1, 10, 11};
-    for (uint32_t k = 0; k < 4; k++)
-      if ((q >> k) & 1u) b = qm_mul(b, factor_or_one(factors, max_log_n, bits[k]));
-  } else if (q < 20) {
-    for (uint32_t k = 0; k < 2; k++)
-      if (((q - 16) >> k) & 1u) b = qm_mul(b, factor_or_one(factors, max_log_n, 12 + k));
-  } else if (q < 28) {
-    b = factor_or_one(factors, max_log_n, 2 + (q - 20));
-  } else {
+// One entry per lane; blockIdx.y = point.
+__global__ __launch_bounds__(EV_WG) void k_eval_tables(const uint32_t* factors, uint32_t max_log_n, EvalTables T,
+                                                       uint32_t* tables) {
+  const uint32_t pt = blockIdx.y;
+  uint32_t x = blockIdx.x * EV_WG + threadIdx.x;
+  factors += (uint64_t)pt * 4 * (max_log_n ? max_log_n : 1);
+  qm31* out = reinterpret_cast<qm31*>(tables);
+  const qm31 one{{1u, 0u, 0u, 0u}};
+  qm31 b = one;
+  if (x <= EV_TERMS) {  // E[x], or C = 2^30 times their sum, the product of 1 + F over the bits
+#pragma unroll
+    for (uint32_t k = 0; k < 6; k++) {
+      const qm31 f = factor_or_one(factors, max_log_n, k < 2 ? k : 8 + k);
+      if (x == EV_TERMS) b = qm_mul(b, qm_add(one, f));
+      else if ((x >> k) & 1u) b = qm_mul(b, f);
+    }
+    if (x == EV_TERMS) {
+      out[T.c() / 4 + pt] = qm_scale(b, 1u << 30);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) b.v[k] = b.v[k] > P / 2 ? b.v[k] - P : b.v[k];
+      out[T.e() / 4 + x * T.np + pt] = b;
+    }
     return;
   }
-  reinterpret_cast<qm31*>(table)[q] = b;
-}
-
-// 256-lane LDS fold of q[0..256) with the factors f[0..8) (uniform).
-__device__ qm31 lds_fold_table(qm31* q, qm31 v, uniform_t<qm31>* f) {
-  const uint32_t t = threadIdx.x;
-  q[t] = v;
-  __syncthreads();
+  x -= EV_TERMS + 1;
+  if (x < EV_WG) {
 #pragma unroll
-  for (uint32_t j = 0; j < EV_WG_LOG; j++) {
-    const qm31 fj{{f[j].v[0], f[j].v[1], f[j].v[2], f[j].v[3]}};
-    if ((t & ((2u << j) - 1)) == 0) q[t] = qm_add(q[t], qm_mul(fj, q[t + (1u << j)]));
-    __syncthreads();
+    for (uint32_t k = 0; k < EV_WG_LOG; k++)
+      if ((x >> k) & 1u) b = qm_mul(b, factor_or_one(factors, max_log_n, 2 + k));
+    out[T.l() / 4 + pt * EV_WG + x] = b;
+    return;
   }
-  return q[0];
+  x -= EV_WG;
+  if (x >> T.g_log) return;
+  for (uint32_t k = 0; k < T.g_log; k++)
+    if ((x >> k) & 1u) b = qm_mul(b, ld_factor(factors, max_log_n, EV_BIG_LOG + k));
+  out[T.g() / 4 + ((uint64_t)pt << T.g_log) + x] = b;
 }
 
-// NP points (1, or 2 for the OODS step's z and z_next) from one read of the
-// coefficients: table holds NP 28-entry tables, part NP arrays of
-// part_stride QM31.
+// lo + 2 hi, congruent mod P: below 2^33 in absolute value for any x. One
+// v_mad_i64_i32 (see m31_fold64).
+__device__ __forceinline__ int64_t fold_signed(int64_t x) {
+  int32_t two = 2;
+  asm("" : "+s"(two));
+  return (int64_t)(int32_t)(x >> 32) * two + (uint32_t)x;
+}
+__device__ __forceinline__ uint32_t wave_sum_mod_p(uint32_t v) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) v = m31_add(v, (uint32_t)__shfl_xor((int)v, off, 64));
+  return v;
+}
+
 template <uint32_t NP>
-__global__ __launch_bounds__(EV_WG) void k_eval_batch_chunks(const EvalChunkJob* jobs, uint32_t n_jobs,
-                                                             const uint32_t* table, uint32_t* part,
-                                                             uint32_t part_stride) {
-  __shared__ qm31 q[EV_WG];
-  const uint32_t b = blockIdx.x, t = threadIdx.x;
-  uint32_t lo = 0, hi = n_jobs;
+__global__ __launch_bounds__(EV_WG) void k_eval_chunks(EvalCols a, EvalTables T, const uint32_t* tables,
+                                                       uint32_t* part, uint32_t part_stride) {
+  __shared__ qm31 red[NP][EV_WG / 64];
+  const uint32_t wg = blockIdx.x, t = threadIdx.x;
+  uint32_t lo = 0, hi = a.n;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (ld_uniform(&jobs[mid].first_chunk) <= b) lo = mid;
+    if (a.first[mid] <= wg) lo = mid;
     else hi = mid;
   }
-  const uint32_t* col = ld_uniform(&jobs[lo].col);
-  const uint32_t L = ld_uniform(&jobs[lo].log_n);
-  const uint64_t chunk = b - ld_uniform(&jobs[lo].first_chunk);
-  const uint64_t n = 1ull << L;
-  uint4 x[16];
+  const uint32_t* col = a.col[lo];
+  const uint32_t L = a.log_n[lo];
+  const uint32_t n = 1u << L;
+  const uint32_t chunks = L > EV_BIG_LOG ? 1u << (L - EV_BIG_LOG) : 1u;
+  const uint32_t c0 = (wg - a.first[lo]) << a.cpw_log, c1 = min(c0 + (1u << a.cpw_log), chunks);
+  qm31 sum[NP];
 #pragma unroll
-  for (uint32_t m = 0; m < 16; m++) {
-    const uint64_t w = (chunk << EV_BIG_LOG) + 4ull * (t + m * EV_WG);  // first word of the load
-    if (L >= 2) {
-      x[m] = w < n ? reinterpret_cast<const uint4*>(col)[w >> 2] : make_uint4(0u, 0u, 0u, 0u);
-    } else {
-      x[m] = make_uint4(w < n ? col[w] : 0u, w + 1 < n ? col[w + 1] : 0u, 0u, 0u);
+  for (uint32_t pt = 0; pt < NP; pt++) sum[pt] = qm31{{0u, 0u, 0u, 0u}};
+#pragma unroll 1
+  for (uint32_t chunk = c0; chunk < c1; chunk++) {
+    // load m of this lane: words w, w + 1, ... of the column (zero past its end)
+    auto load = [&](uint32_t m) {
+      const uint32_t w = 4 * (t + m * EV_WG);
+      if (L >= EV_BIG_LOG) return *reinterpret_cast<const uint4*>(col + ((uint64_t)chunk << EV_BIG_LOG) + w);
+      if (L >= 2) return w < n ? *reinterpret_cast<const uint4*>(col + w) : make_uint4(0u, 0u, 0u, 0u);
+      return make_uint4(w < n ? col[w] : 0u, w + 1 < n ? col[w + 1] : 0u, 0u, 0u);
+    };
+    int64_t acc[NP][4];
+#pragma unroll
+    for (uint32_t pt = 0; pt < NP; pt++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) acc[pt][k] = 0;
+    uniform_t<int32_t>* E = (uniform_t<int32_t>*)(tables + T.e());
+    uint4 x[2] = {load(0), load(1)};
+    // A loop, not unrolled: the weights of a step fill 64 scalar registers, and
+    // unrolled the compiler reads those of all steps ahead and spills them.
+#pragma unroll 1
+    for (uint32_t m = 0; m < 16; m += 2) {
+      const uint4 y[2] = {x[0], x[1]};
+      if (m < 14) {
+        x[0] = load(m + 2);
+        x[1] = load(m + 3);
+      }
+#pragma unroll
+      for (uint32_t h = 0; h < 2; h++) {
+        const uint32_t xv[4] = {y[h].x, y[h].y, y[h].z, y[h].w};
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) {
+          const int64_t xs = (int32_t)(xv[r] - (1u << 30));
+#pragma unroll
+          for (uint32_t pt = 0; pt < NP; pt++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) acc[pt][k] += xs * E[4 * (NP * (4 * h + r) + pt) + k];
+        }
+      }
+      E += 4 * NP * 8;
+      // eight products of at most 2^30 (2^30 - 1) and a folded sum stay below 2^63
+#pragma unroll
+      for (uint32_t pt = 0; pt < NP; pt++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[pt][k] = fold_signed(acc[pt][k]);
+    }
+#pragma unroll
+    for (uint32_t pt = 0; pt < NP; pt++) {
+      const qm31 C = ld_uniform(reinterpret_cast<const qm31*>(tables + T.c()) + pt);
+      qm31 s;
+#pragma unroll
+      for (int k = 0; k < 4; k++) s.v[k] = m31_reduce64((uint64_t)(acc[pt][k] + ((int64_t)P << 3)) + C.v[k]);
+      if (chunk != 0) {  // G[0] = 1
+        const qm31_mat g =
+            qm_left_matrix(ld_uniform(reinterpret_cast<const qm31*>(tables + T.g()) + ((uint64_t)pt << T.g_log) + chunk));
+        qm31 r;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          r.v[k] = m31_reduce64((uint64_t)g.m[k][0] * s.v[0] + (uint64_t)g.m[k][1] * s.v[1] +
+                                (uint64_t)g.m[k][2] * s.v[2] + (uint64_t)g.m[k][3] * s.v[3]);
+        s = r;
+      }
+      sum[pt] = qm_add(sum[pt], s);
     }
   }
 #pragma unroll
   for (uint32_t pt = 0; pt < NP; pt++) {
-    const uint32_t* tab = table + 28 * 4 * pt;
-    uniform_t<qm31>* E = (uniform_t<qm31>*)tab;
-    qm31 w4[4];
+    const uint4 lv = reinterpret_cast<const uint4*>(tables + T.l())[pt * EV_WG + t];
+    qm31 s = qm_mul_lazy(qm31{{lv.x, lv.y, lv.z, lv.w}}, sum[pt]);
 #pragma unroll
-    for (uint32_t m23 = 0; m23 < 4; m23++) {
-#pragma unroll
-      for (uint32_t k = 0; k < 4; k++) {
-        uint32_t r = 0;
-#pragma unroll
-        for (uint32_t m01 = 0; m01 < 4; m01++) {
-          const uint4 v = x[m01 + 4 * m23];
-          const uint64_t acc = (uint64_t)v.x * E[4 * m01].v[k] + (uint64_t)v.y * E[4 * m01 + 1].v[k] +
-                               (uint64_t)v.z * E[4 * m01 + 2].v[k] + (uint64_t)v.w * E[4 * m01 + 3].v[k];
-          r = m31_add(r, m31_reduce64(acc));
-        }
-        w4[m23].v[k] = r;
-      }
-    }
-    qm31 v = w4[0];
-#pragma unroll
-    for (uint32_t m23 = 1; m23 < 4; m23++)
-      v = qm_add(v, qm_mul(ld_uniform(reinterpret_cast<const qm31*>(tab) + 16 + m23), w4[m23]));
-    const qm31 sum = lds_fold_table(q, v, (uniform_t<qm31>*)tab + 20);
-    if (t == 0) reinterpret_cast<qm31*>(part)[(uint64_t)pt * part_stride + b] = sum;
-    if (NP > 1) __syncthreads();  // q is reused by the next point's fold
+    for (int k = 0; k < 4; k++) s.v[k] = wave_sum_mod_p(s.v[k]);
+    if ((t & 63) == 0) red[pt][t >> 6] = s;
   }
-}
-
-// blockIdx.y = point: its factors, input and output arrays lie f_stride,
-// in_stride and out_stride words after the previous point's.
-__global__ __launch_bounds__(EV_WG) void k_eval_batch_fold(const EvalFoldJob* jobs, const uint32_t* factors,
-                                                           uint32_t max_log_n, const uint32_t* in, uint32_t* out,
-                                                           uint32_t f_stride, uint32_t in_stride,
-                                                           uint32_t out_stride) {
-  __shared__ qm31 q[EV_WG];
-  const uint32_t t = threadIdx.x;
-  factors += (uint64_t)blockIdx.y * f_stride;
-  in += (uint64_t)blockIdx.y * in_stride;
-  out += (uint64_t)blockIdx.y * out_stride;
-  uniform_t<EvalFoldJob>& J = as_uniform(jobs + blockIdx.x);
-  const uint32_t n = J.n, fb = J.fb;
-  qm31 f[EV_WG_LOG];
-#pragma unroll
-  for (uint32_t j = 0; j < EV_WG_LOG; j++) f[j] = factor_or_one(factors, max_log_n, fb + j);
-  q[t] = t < n ? reinterpret_cast<const qm31*>(in)[J.in + t] : qm31{{0u, 0u, 0u, 0u}};
   __syncthreads();
-#pragma unroll
-  for (uint32_t j = 0; j < EV_WG_LOG; j++) {
-    if ((t & ((2u << j) - 1)) == 0) q[t] = qm_add(q[t], qm_mul(f[j], q[t + (1u << j)]));
-    __syncthreads();
+  if (t < NP) {
+    qm31 s = red[t][0];
+    for (uint32_t w = 1; w < EV_WG / 64; w++) s = qm_add(s, red[t][w]);
+    reinterpret_cast<qm31*>(part)[(uint64_t)t * part_stride + a.wg_base + wg] = s;
   }
-  if (t == 0) reinterpret_cast<qm31*>(out)[J.out] = q[0];
 }
 
-// result[k] = QM31 at src[k] (device pointers, one per column)
-__global__ void k_copy_qm31(const uint32_t* const* src, uint32_t* results, uint32_t n) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  reinterpret_cast<qm31*>(results)[k] = *reinterpret_cast<const qm31*>(src[k]);
+// results[pt * n_cols + col_base + k] = the sum of column k's workgroups'
+// sums; one wavefront per (column, point).
+__global__ __launch_bounds__(64) void k_eval_sum(EvalCols a, uint32_t n_wgs, const uint32_t* part,
+                                                 uint32_t part_stride, uint32_t* results, uint32_t n_cols,
+                                                 uint32_t col_base) {
+  const uint32_t k = blockIdx.x, pt = blockIdx.y, lane = threadIdx.x;
+  const uint32_t b = a.first[k], e = k + 1 < a.n ? a.first[k + 1] : n_wgs;
+  const qm31* p = reinterpret_cast<const qm31*>(part) + (uint64_t)pt * part_stride + a.wg_base;
+  uint64_t s[4] = {0, 0, 0, 0};
+  for (uint32_t i = b + lane; i < e; i += 64)
+#pragma unroll
+    for (int c = 0; c < 4; c++) s[c] += p[i].v[c];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const uint32_t v = wave_sum_mod_p(m31_reduce64(s[c]));
+    if (lane == 0) results[4 * ((uint64_t)pt * n_cols + col_base + k) + c] = v;
+  }
 }
 
 // np points (1 or 2): factors holds np tables of 4 max_log_n words back to
 // back (4 words when max_log_n is 0), results np arrays of n_cols QM31.
+// The work is enqueued on s; `ws` is the caller's to free when it is done.
 static void eval_batch_points(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
                               const uint32_t* factors, uint32_t np, uint32_t max_log_n, uint32_t* results,
-                              hipStream_t s) {
+                              DeviceBuf& ws, hipStream_t s) {
   if (n_cols == 0) return;
   require(np == 1 || np == 2, "eval_at_point_batch: one or two points");
-  const uint32_t f_stride = 4 * (max_log_n ? max_log_n : 1);
   require(max_log_n <= 31, "eval_at_point_batch: max_log_n must be <= 31");
-  std::vector<EvalChunkJob> jobs(n_cols);
-  std::vector<uint32_t> count(n_cols), off(n_cols);
   uint64_t total = 0;
+  uint32_t top = 0;
   for (uint32_t k = 0; k < n_cols; k++) {
     const uint32_t L = h_log_sizes[k];
     require(h_cols[k] != nullptr && L <= max_log_n, "eval_at_point_batch: null column or log size above max_log_n");
     require(L < 2 || (reinterpret_cast<uintptr_t>(h_cols[k]) & 15u) == 0,
             "eval_at_point_batch: columns must be 16-byte aligned");
-    count[k] = L > EV_BIG_LOG ? 1u << (L - EV_BIG_LOG) : 1u;
-    off[k] = (uint32_t)total;
-    jobs[k] = {h_cols[k], L, (uint32_t)total};
-    total += count[k];
+    total += L > EV_BIG_LOG ? 1ull << (L - EV_BIG_LOG) : 1ull;
+    top = L > top ? L : top;
   }
   require(total < (1ull << 31), "eval_at_point_batch: too many chunks");
-  // every level's sums stay allocated until the results are copied: a column
-  // that is down to one sum keeps it where it was written
-  std::vector<DeviceBuf> keep;
-  keep.emplace_back(sizeof(EvalChunkJob) * n_cols);
-  VX_HIP(hipMemcpyAsync(keep.back().p, jobs.data(), sizeof(EvalChunkJob) * n_cols, hipMemcpyHostToDevice, s));
-  const EvalChunkJob* d_jobs = static_cast<const EvalChunkJob*>(keep.back().p);
-  keep.emplace_back(np * 28 * 16);
-  uint32_t* d_table = keep.back().u32();
-  keep.emplace_back(np * total * 16);
-  uint32_t* level = keep.back().u32();
-  uint32_t level_stride = 4 * (uint32_t)total;  // words between the points' arrays
-  for (uint32_t pt = 0; pt < np; pt++)
-    hipLaunchKernelGGL(k_eval_batch_setup, dim3(1), dim3(64), 0, s, factors + pt * f_stride, max_log_n,
-                       d_table + 28 * 4 * pt);
-  if (np == 2)
-    hipLaunchKernelGGL(k_eval_batch_chunks<2>, dim3((uint32_t)total), dim3(EV_WG), 0, s, d_jobs, n_cols, d_table,
-                       level, (uint32_t)total);
-  else
-    hipLaunchKernelGGL(k_eval_batch_chunks<1>, dim3((uint32_t)total), dim3(EV_WG), 0, s, d_jobs, n_cols, d_table,
-                       level, (uint32_t)total);
-  VX_HIP(hipGetLastError());
-  // final_src[pt * n_cols + k]: where column k's sum for point pt ends up
-  std::vector<const uint32_t*> final_src((size_t)np * n_cols, nullptr);
-  auto settle = [&](uint32_t k, const uint32_t* lv, uint32_t stride) {
-    for (uint32_t pt = 0; pt < np; pt++) final_src[(size_t)pt * n_cols + k] = lv + (uint64_t)pt * stride + 4ull * off[k];
+  // Chunks per workgroup: the lanes' products by L and their sum are paid
+  // once per workgroup, so no more workgroups than keep the chip full.
+  uint32_t cpw_log = 0;
+  while ((total >> cpw_log) > EV_MAX_WGS) cpw_log++;
+  auto wgs_of = [&](uint32_t L) {
+    const uint32_t c = L > EV_BIG_LOG ? L - EV_BIG_LOG : 0;
+    return c > cpw_log ? 1u << (c - cpw_log) : 1u;
   };
-  for (uint32_t k = 0; k < n_cols; k++)
-    if (count[k] == 1) settle(k, level, level_stride);
-  uint32_t fb = EV_BIG_LOG;
-  for (;;) {
-    std::vector<EvalFoldJob> fj;
-    uint32_t next = 0;
-    for (uint32_t k = 0; k < n_cols; k++) {
-      if (count[k] <= 1) continue;
-      const uint32_t w = count[k] < EV_WG ? count[k] : EV_WG;
-      const uint32_t groups = count[k] / w;
-      for (uint32_t g = 0; g < groups; g++) fj.push_back({off[k] + g * w, next + g, w, fb});
-      off[k] = next;
-      count[k] = groups;
-      next += groups;
-    }
-    if (fj.empty()) break;
-    keep.emplace_back(sizeof(EvalFoldJob) * fj.size());
-    VX_HIP(hipMemcpyAsync(keep.back().p, fj.data(), sizeof(EvalFoldJob) * fj.size(), hipMemcpyHostToDevice, s));
-    const EvalFoldJob* d_fj = static_cast<const EvalFoldJob*>(keep.back().p);
-    keep.emplace_back((size_t)np * next * 16);
-    uint32_t* out = keep.back().u32();
-    hipLaunchKernelGGL(k_eval_batch_fold, dim3((uint32_t)fj.size(), np), dim3(EV_WG), 0, s, d_fj, factors,
-                       max_log_n, level, out, f_stride, level_stride, 4 * next);
-    VX_HIP(hipGetLastError());
-    level = out;
-    level_stride = 4 * next;
-    for (uint32_t k = 0; k < n_cols; k++)
-      if (count[k] == 1 && final_src[k] == nullptr) settle(k, level, level_stride);
-    fb += EV_WG_LOG;
-  }
-  const uint32_t n_out = np * n_cols;
-  keep.emplace_back(sizeof(uint32_t*) * n_out);
-  VX_HIP(hipMemcpyAsync(keep.back().p, final_src.data(), sizeof(uint32_t*) * n_out, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_copy_qm31, dim3((n_out + 255) / 256), dim3(256), 0, s,
-                     static_cast<const uint32_t* const*>(keep.back().p), results, n_out);
+  uint64_t wgs = 0;
+  for (uint32_t k = 0; k < n_cols; k++) wgs += wgs_of(h_log_sizes[k]);
+  const EvalTables T{np, top > EV_BIG_LOG ? top - EV_BIG_LOG : 0};
+  ws = DeviceBuf(4 * T.words() + 16ull * np * wgs);
+  uint32_t* tables = ws.u32();
+  uint32_t* part = tables + T.words();
+  const uint64_t entries = EV_TERMS + 1 + EV_WG + (1ull << T.g_log);
+  hipLaunchKernelGGL(k_eval_tables, dim3((uint32_t)((entries + EV_WG - 1) / EV_WG), np), dim3(EV_WG), 0, s, factors,
+                     max_log_n, T, tables);
   VX_HIP(hipGetLastError());
-  // the staging buffers are freed on return: the caller's stream must be done
-  VX_HIP(hipStreamSynchronize(s));
+  uint32_t wg_base = 0;
+  for (uint32_t k0 = 0; k0 < n_cols; k0 += EV_ARG_COLS) {
+    EvalCols a{};
+    a.n = n_cols - k0 < EV_ARG_COLS ? n_cols - k0 : EV_ARG_COLS;
+    a.cpw_log = cpw_log;
+    a.wg_base = wg_base;
+    uint32_t w = 0;
+    for (uint32_t k = 0; k < a.n; k++) {
+      a.col[k] = h_cols[k0 + k];
+      a.log_n[k] = (uint8_t)h_log_sizes[k0 + k];
+      a.first[k] = w;
+      w += wgs_of(h_log_sizes[k0 + k]);
+    }
+    if (np == 2)
+      hipLaunchKernelGGL(k_eval_chunks<2>, dim3(w), dim3(EV_WG), 0, s, a, T, tables, part, (uint32_t)wgs);
+    else
+      hipLaunchKernelGGL(k_eval_chunks<1>, dim3(w), dim3(EV_WG), 0, s, a, T, tables, part, (uint32_t)wgs);
+    VX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_eval_sum, dim3(a.n, np), dim3(64), 0, s, a, w, part, (uint32_t)wgs, results, n_cols, k0);
+    VX_HIP(hipGetLastError());
+    wg_base += w;
+  }
 }
 
 void eval_at_point_batch(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
                          const uint32_t* factors, uint32_t max_log_n, uint32_t* results, hipStream_t s) {
-  eval_batch_points(h_cols, h_log_sizes, n_cols, factors, 1, max_log_n, results, s);
+  DeviceBuf ws;
+  eval_batch_points(h_cols, h_log_sizes, n_cols, factors, 1, max_log_n, results, ws, s);
+  VX_HIP(hipStreamSynchronize(s));  // the workspace is freed on return
 }
 
 // ---------------------------------------------------------------------------
@@ -521,22 +561,28 @@ __device__ void oods_factors(qm31 zx, qm31 zy, uint32_t max_log, uint32_t* out) 
   for (uint32_t i = 0; i < max_log; i++) {
     const qm31 m = i == 0 ? zy : x;
     if (i > 0) {
-      const qm31 x2 = qm_mul(x, x);
+      const qm31 x2 = qm_mul_lazy(x, x);
       x = qm_sub(qm_add(x2, x2), qm31{{1u, 0u, 0u, 0u}});
     }
     for (int k = 0; k < 4; k++) out[4 * (max_log - 1 - i) + k] = m.v[k];
   }
 }
 
+// A dependent chain on one lane: the draw, the division, then max_log
+// doublings. Lane 0 follows z and lane 1 z_next (both draw z), so the two
+// chains of doublings run side by side: 22 -> 14 us for max_log 20.
 __global__ void k_oods_point(uint32_t* ch_words, uint32_t trace_log, uint32_t max_log, uint32_t* points, uint32_t* fz,
                              uint32_t* fzn) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  if (threadIdx.x > 1 || blockIdx.x != 0) return;
+  const bool next = threadIdx.x == 1;
   Channel c;
   for (int i = 0; i < 8; i++) c.state[i] = ch_words[i];
   c.n_draws = ch_words[8];
   const qm31 t = ch_draw_felt(c);
-  for (int i = 0; i < 8; i++) ch_words[i] = c.state[i];
-  ch_words[8] = c.n_draws;
+  if (!next) {
+    for (int i = 0; i < 8; i++) ch_words[i] = c.state[i];
+    ch_words[8] = c.n_draws;
+  }
   const qm31 one{{1u, 0u, 0u, 0u}};
   const qm31 t2 = qm_mul(t, t);
   const qm31 inv = qm_inv(qm_add(one, t2));
@@ -544,36 +590,39 @@ __global__ void k_oods_point(uint32_t* ch_words, uint32_t trace_log, uint32_t ma
   const cpt st = c_rdouble(c_generator(), 31 - trace_log);
   const qm31 nx = qm_sub(qm_scale(zx, st.x), qm_scale(zy, st.y));
   const qm31 ny = qm_add(qm_scale(zx, st.y), qm_scale(zy, st.x));
-  const qm31 pts[4] = {zx, zy, nx, ny};
-  for (int p = 0; p < 4; p++)
-    for (int k = 0; k < 4; k++) points[4 * p + k] = pts[p].v[k];
-  oods_factors(zx, zy, max_log, fz);
-  oods_factors(nx, ny, max_log, fzn);
+  const qm31 px = next ? nx : zx, py = next ? ny : zy;
+  for (int k = 0; k < 4; k++) {
+    points[(next ? 8 : 0) + k] = px.v[k];
+    points[(next ? 12 : 4) + k] = py.v[k];
+  }
+  oods_factors(px, py, max_log, next ? fzn : fz);
 }
 
 // Channel::mix_felts (src/channel.rs:46-59) of the sampled values: the
-// message is state || values, values being msg[8..] (msg[0..8) unused); it
-// is a dependent chain of compressions, which the four lanes of a quad
-// share (b2_compress_x4, about 440 instructions per lane and block instead
-// of 960). One wavefront; lanes 0..3 write the new state.
-__global__ __launch_bounds__(64) void k_oods_mix(uint32_t* ch_words, const uint32_t* msg, uint32_t n_felts) {
+// message is state || values; it is a dependent chain of compressions, which
+// the four lanes of a quad share (b2_compress_x4, about 430 instructions per
+// lane and block instead of 960). A block's words are loaded while the block
+// before it is compressed. One wavefront; lanes 0..3 write the new state.
+__global__ __launch_bounds__(64) void k_oods_mix(uint32_t* ch_words, const uint32_t* values, uint32_t n_felts) {
   if (blockIdx.x != 0 || n_felts == 0) return;
   const uint32_t q = threadIdx.x & 3u;
   const bool q0 = q & 1, q1 = q & 2;
   uint32_t h_lo = sel4(q0, q1, VX_B2_IV0 ^ 0x01010020u, VX_B2_IV1, VX_B2_IV2, VX_B2_IV3);
   uint32_t h_hi = sel4(q0, q1, VX_B2_IV4, VX_B2_IV5, VX_B2_IV6, VX_B2_IV7);
-  const uint32_t nbytes = 32u + 16u * n_felts;
-  for (uint32_t off = 0;; off += 64) {
-    const uint32_t rem = nbytes - off;
-    const bool last = rem <= 64;
-    uint32_t m[16];
+  const uint32_t nwords = 8 + 4 * n_felts;
+  uint32_t m[16], next[16];
 #pragma unroll
-    for (uint32_t k = 0; k < 16; k++) {
-      const uint32_t w = off / 4 + k;
-      m[k] = 4 * k < rem ? (w < 8 ? ch_words[w] : msg[w]) : 0u;
+  for (uint32_t k = 0; k < 16; k++) m[k] = k < 8 ? ch_words[k] : k < nwords ? values[k - 8] : 0u;
+  for (uint32_t at = 0;; at += 16) {
+    const bool last = nwords - at <= 16;
+    if (!last) {
+#pragma unroll
+      for (uint32_t k = 0; k < 16; k++) next[k] = at + 16 + k < nwords ? values[at + 8 + k] : 0u;
     }
-    b2_compress_x4(h_lo, h_hi, m, last ? nbytes : off + 64, last, q);
+    b2_compress_x4(h_lo, h_hi, m, last ? 4 * nwords : 4 * (at + 16), last, q);
     if (last) break;
+#pragma unroll
+    for (uint32_t k = 0; k < 16; k++) m[k] = next[k];
   }
   if (threadIdx.x < 4) {
     ch_words[q] = h_lo;
@@ -587,19 +636,17 @@ void oods_sample(uint32_t* d_channel, const uint32_t* const* h_cols, const uint3
   uint32_t max_log = 0;
   for (uint32_t k = 0; k < n_cols; k++) max_log = h_log_sizes[k] > max_log ? h_log_sizes[k] : max_log;
   const uint32_t fw = 4 * (max_log ? max_log : 1);
-  DeviceBuf fac(8ull * fw), msg(4ull * (8 + 8ull * n_cols));
-  uint32_t* fz = static_cast<uint32_t*>(fac.p);
-  uint32_t* m = static_cast<uint32_t*>(msg.p);
+  DeviceBuf fac(8ull * fw), ws;
+  uint32_t* fz = fac.u32();
   hipLaunchKernelGGL(k_oods_point, dim3(1), dim3(64), 0, s, d_channel, trace_log, max_log, d_points, fz, fz + fw);
   VX_HIP(hipGetLastError());
   if (n_cols) {
     // both points from one read of every column: values at z, then at z_next
-    eval_batch_points(h_cols, h_log_sizes, n_cols, fz, 2, max_log, m + 8, s);
-    hipLaunchKernelGGL(k_oods_mix, dim3(1), dim3(64), 0, s, d_channel, m, 2 * n_cols);
+    eval_batch_points(h_cols, h_log_sizes, n_cols, fz, 2, max_log, d_values, ws, s);
+    hipLaunchKernelGGL(k_oods_mix, dim3(1), dim3(64), 0, s, d_channel, d_values, 2 * n_cols);
     VX_HIP(hipGetLastError());
-    VX_HIP(hipMemcpyAsync(d_values, m + 8, 32ull * n_cols, hipMemcpyDeviceToDevice, s));
   }
-  VX_HIP(hipStreamSynchronize(s));
+  VX_HIP(hipStreamSynchronize(s));  // the workspaces are freed on return
 }
 
 }  // namespace vx
