@@ -5,6 +5,7 @@
 // mixed by a single lane, and the next fold reads its alpha from device
 // memory. Query draws are independent squeezes (n_draws = 0..nq-1 after
 // mix_felts), so one lane per query computes them in parallel.
+#include "vx_blake2s_wide.h"
 #include "vx_internal.h"
 
 namespace vx {
@@ -105,11 +106,20 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
 // map that keeps the order, so the smallest index is the smallest nonce.
 __device__ __forceinline__ uint64_t stwo_nonce(uint64_t i) { return ((i >> 20) << 32) | (i & 0xFFFFFull); }
 
-template <bool STWO, bool M31_OUT = false>
+// WIDE (grids of at least two wavefronts per SIMD): b2_compress_wide's half
+// rounds. The first one mixes the prefix only, so it is done once per lane
+// and not per nonce. PoW 20 (about 2^20 nonces, 1,024 workgroups): 20.0 ->
+// 17.9 us.
+template <bool STWO, bool M31_OUT, bool WIDE>
 __global__ __launch_bounds__(256) void k_grind(const uint32_t* prefix_dev, uint32_t bits,
                                               unsigned long long* best, uint64_t start, uint64_t count) {
   uint32_t prefix[8];
   for (int k = 0; k < 8; k++) prefix[k] = prefix_dev[k];
+  uint32_t h0[8], v0[16];
+  b2_init(h0);
+  b2_state(v0, h0, 40u, true);
+#pragma unroll
+  for (int i = 0; i < 4; i++) VX_B2_G(v0[i], v0[4 + i], v0[8 + i], v0[12 + i], prefix[2 * i], prefix[2 * i + 1]);
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   const uint64_t end = start + count;
   for (uint64_t base = start + (uint64_t)blockIdx.x * blockDim.x; base < end; base += stride) {
@@ -120,11 +130,37 @@ __global__ __launch_bounds__(256) void k_grind(const uint32_t* prefix_dev, uint3
                               (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)seen);
     if (base > cur_best) break;
     const uint64_t n = base + threadIdx.x;
+    const uint64_t nonce = STWO ? stwo_nonce(n) : n;
+    uint32_t tz;
+    if constexpr (WIDE) {
+      const uint32_t m[16] = {prefix[0], prefix[1], prefix[2], prefix[3],     prefix[4],
+                              prefix[5], prefix[6], prefix[7], (uint32_t)nonce, (uint32_t)(nonce >> 32)};
+      uint32_t v[16], h[4];
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = v0[i];
+      b2_rounds_wide<10, 1>(v, m);
+#pragma unroll
+      for (int i = 0; i < 4; i++) h[i] = h0[i] ^ v[i] ^ v[8 + i];
+      tz = digest_trailing_zeros<M31_OUT>(h);
+    } else {
+      tz = pow_trailing_zeros<M31_OUT>(prefix, nonce);
+    }
     uint64_t hit = ~0ull;
-    if (n < end && pow_trailing_zeros<M31_OUT>(prefix, STWO ? stwo_nonce(n) : n) >= bits) hit = n;
+    if (n < end && tz >= bits) hit = n;
     hit = wave_min_u64(hit);
     if ((threadIdx.x & 63) == 0 && hit != ~0ull) atomicMin(best, (unsigned long long)hit);
   }
+}
+
+// 512 workgroups of 256 lanes are two wavefronts per SIMD of 256 CUs.
+template <bool STWO>
+static void launch_grind(uint32_t grid, bool m31_out, const uint32_t* prefix, uint32_t bits, unsigned long long* best,
+                         uint64_t start, uint64_t count, hipStream_t s) {
+  const bool wide = grid >= 512;
+  hipLaunchKernelGGL(m31_out ? (wide ? k_grind<STWO, true, true> : k_grind<STWO, true, false>)
+                             : (wide ? k_grind<STWO, false, true> : k_grind<STWO, false, false>),
+                     dim3(grid), dim3(256), 0, s, prefix, bits, best, start, count);
+  VX_HIP(hipGetLastError());
 }
 
 __global__ void k_set_u64(unsigned long long* p, unsigned long long v) {
@@ -154,12 +190,7 @@ void grind_pow_stwo(const uint32_t* d_prefix, uint32_t pow_bits, uint64_t* d_res
   require(pow_bits >= 1 && pow_bits <= 32, "grind_pow_stwo: pow_bits must be 1..32");
   auto* best = reinterpret_cast<unsigned long long*>(d_result);
   hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(64), 0, s, best, ~0ull);
-  if (m31_out)
-    hipLaunchKernelGGL((k_grind<true, true>), dim3(grind_grid(pow_bits)), dim3(256), 0, s, d_prefix, pow_bits, best,
-                       0ull, GRIND_LIMIT);
-  else
-    hipLaunchKernelGGL((k_grind<true, false>), dim3(grind_grid(pow_bits)), dim3(256), 0, s, d_prefix, pow_bits,
-                       best, 0ull, GRIND_LIMIT);
+  launch_grind<true>(grind_grid(pow_bits), m31_out, d_prefix, pow_bits, best, 0ull, GRIND_LIMIT, s);
   hipLaunchKernelGGL(k_stwo_index_to_nonce, dim3(1), dim3(64), 0, s, best);
   VX_HIP(hipGetLastError());
 }
@@ -169,9 +200,7 @@ void grind_pow(const uint32_t* d_prefix, uint32_t pow_bits, uint64_t* d_result, 
   auto* best = reinterpret_cast<unsigned long long*>(d_result);
   hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(64), 0, s, best, ~0ull);
   // every lane loops until its nonce exceeds the best hit
-  hipLaunchKernelGGL(k_grind<false>, dim3(grind_grid(pow_bits)), dim3(256), 0, s, d_prefix, pow_bits, best, 0ull,
-                     GRIND_LIMIT);
-  VX_HIP(hipGetLastError());
+  launch_grind<false>(grind_grid(pow_bits), false, d_prefix, pow_bits, best, 0ull, GRIND_LIMIT, s);
 }
 
 // Reference-style batch (cuda/grind.cu:94-110): test nonces
@@ -182,13 +211,7 @@ void grind_pow_batch(const uint32_t* d_prefix, uint64_t* d_result, uint32_t pow_
   uint64_t blocks = (n + 255) / 256;
   uint32_t grid = (uint32_t)(blocks < 4096 ? blocks : 4096);
   auto* best = reinterpret_cast<unsigned long long*>(d_result);
-  if (m31_out)
-    hipLaunchKernelGGL((k_grind<false, true>), dim3(grid), dim3(256), 0, s, d_prefix, pow_bits, best, batch_offset,
-                       n);
-  else
-    hipLaunchKernelGGL((k_grind<false, false>), dim3(grid), dim3(256), 0, s, d_prefix, pow_bits, best, batch_offset,
-                       n);
-  VX_HIP(hipGetLastError());
+  launch_grind<false>(grid, m31_out, d_prefix, pow_bits, best, batch_offset, n, s);
 }
 
 struct WordWrites {

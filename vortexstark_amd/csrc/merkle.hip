@@ -22,7 +22,11 @@
 // hashed. The kernel that produces a root also runs the transcript step
 // (mix the root, draw the next alpha), so no separate channel launch is
 // needed. FRI layers of <= 2^10 values are committed by one workgroup in a
-// single launch (k_fri_tail). Blake2s is VALU-bound here.
+// single launch (k_fri_tail). Blake2s is VALU-bound here: the kernels that run
+// several wavefronts per SIMD use the form whose wavefronts issue together
+// (b2_compress_wide), those that are one wavefront's dependent chain
+// b2_compress and the quad forms.
+#include "vx_blake2s_wide.h"
 #include "vx_blake2s_x4.h"
 #include "vx_channel_x4.h"
 #include "vx_d2.h"
@@ -268,8 +272,13 @@ __device__ __forceinline__ void lifted_block(const LiftCol* cols, uint32_t n, ui
     }
   }
 }
+template <bool WIDE>
 __device__ __forceinline__ void lifted_leaf_cols(const LiftCol* cols, uint32_t n, uint32_t S, uint64_t idx,
-                                                 uint32_t h[8]) {
+                                                 uint32_t (&h)[8]) {
+  auto compress = [&](const uint32_t (&m)[16], uint32_t t, bool last) {
+    if constexpr (WIDE) b2_compress_wide(h, m, t, last);
+    else b2_compress(h, m, t, last);
+  };
   b2_init(h);
   if (S <= 30) {
     // rows and byte offsets fit 32 bits. (Loading the next block before
@@ -280,7 +289,7 @@ __device__ __forceinline__ void lifted_leaf_cols(const LiftCol* cols, uint32_t n
       uint32_t m[16];
       const bool more = base + 16 < n;
       lifted_block(cols, n, S, i, base, cur, m);
-      b2_compress(h, m, 4 * (more ? base + 16 : n), !more);
+      compress(m, 4 * (more ? base + 16 : n), !more);
     }
     return;
   }
@@ -298,11 +307,12 @@ __device__ __forceinline__ void lifted_leaf_cols(const LiftCol* cols, uint32_t n
       m[j] = v;
     }
     t += 4 * (n - base < 16 ? n - base : 16);
-    b2_compress(h, m, t, base + 16 >= n);
+    compress(m, t, base + 16 >= n);
   }
 }
-__device__ __forceinline__ void lifted_leaf(const LeafSrc& L, uint64_t idx, uint32_t h[8]) {
-  lifted_leaf_cols(L.lift, L.lift_n, L.lift_log, idx, h);
+template <bool WIDE>
+__device__ __forceinline__ void lifted_leaf(const LeafSrc& L, uint64_t idx, uint32_t (&h)[8]) {
+  lifted_leaf_cols<WIDE>(L.lift, L.lift_n, L.lift_log, idx, h);
 }
 
 // Random linear combination of the lifted rows of leaves [i, i+4):
@@ -411,12 +421,35 @@ __device__ __forceinline__ void cairo_readback(const LeafSrc& L, uint64_t i, G4&
   }
 }
 
+// The Blake2s forms by the number of wavefronts that a kernel runs per SIMD.
+template <bool WIDE>
+__device__ __forceinline__ void leaf1(uint32_t x, uint32_t (&h)[8]) {
+  if constexpr (WIDE) b2_leaf1_wide(x, h);
+  else b2_leaf1(x, h);
+}
+template <bool WIDE>
+__device__ __forceinline__ void leaf4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t (&h)[8]) {
+  if constexpr (WIDE) b2_leaf4_wide(a, b, c, d, h);
+  else b2_leaf4(a, b, c, d, h);
+}
+template <bool WIDE>
+__device__ __forceinline__ void hash_words(const uint32_t* w, uint32_t n, uint32_t (&h)[8]) {
+  if constexpr (WIDE) b2_hash_words_wide(w, n, h);
+  else b2_hash_words(w, n, h);
+}
+template <bool WIDE>
+__device__ __forceinline__ void hash_node(const uint32_t* l, const uint32_t* r, uint32_t (&h)[8]) {
+  if constexpr (WIDE) b2_hash_node_wide(l, r, h);
+  else b2_hash_node(l, r, h);
+}
+
 // One leaf per lane: the lane's own row, stored and hashed.
-__device__ __forceinline__ void cairo_leaf(const LeafSrc& L, uint64_t idx, uint32_t out[8]) {
+template <bool WIDE>
+__device__ __forceinline__ void cairo_leaf(const LeafSrc& L, uint64_t idx, uint32_t (&out)[8]) {
   const qm31 q = cairo_row(as_uniform(L.cairo), idx);
 #pragma unroll
   for (int c = 0; c < 4; c++) L.out[c][idx] = q.v[c];
-  b2_leaf4(q.v[0], q.v[1], q.v[2], q.v[3], out);
+  leaf4<WIDE>(q.v[0], q.v[1], q.v[2], q.v[3], out);
 }
 
 // Rows [i, i+4) of up to 16 columns, one 16-byte load per column, all
@@ -429,21 +462,21 @@ __device__ __forceinline__ void cols_load(const LeafSrc& L, uint64_t i, GCols& g
   for (uint32_t c = 0; c < 16; c++) gc.c[c] = c < L.n_cols ? ld4(L.col[c] + i) : make_uint4(0, 0, 0, 0);
 }
 
-template <uint32_t KIND, uint32_t NC>
+template <uint32_t KIND, uint32_t NC, bool WIDE>
 __device__ __forceinline__ void leaf_hash(const LeafSrc& L, const G4& g, const GCols& gc, uint64_t i, int j,
-                                          uint32_t h[8]) {
+                                          uint32_t (&h)[8]) {
   if constexpr (KIND == LEAF_LIFTED) {
-    lifted_leaf(L, i + j, h);
+    lifted_leaf<WIDE>(L, i + j, h);
   } else if constexpr (KIND == LEAF_COLS && NC == 1) {
-    b2_leaf1(g.w[j][0], h);
+    leaf1<WIDE>(g.w[j][0], h);
   } else if constexpr (KIND == LEAF_COLS && NC == 0) {
     // generic 1..16 columns: row i + j of each
     uint32_t w[16];
 #pragma unroll
     for (uint32_t c = 0; c < 16; c++) w[c] = j == 0 ? gc.c[c].x : j == 1 ? gc.c[c].y : j == 2 ? gc.c[c].z : gc.c[c].w;
-    b2_hash_words(w, L.n_cols, h);
+    hash_words<WIDE>(w, L.n_cols, h);
   } else {
-    b2_leaf4(g.w[j][0], g.w[j][1], g.w[j][2], g.w[j][3], h);
+    leaf4<WIDE>(g.w[j][0], g.w[j][1], g.w[j][2], g.w[j][3], h);
   }
 }
 
@@ -453,8 +486,8 @@ __device__ __forceinline__ void cp8(uint32_t d[8], const uint32_t s[8]) {
 }
 
 // Merkle node over the 2^LPT_LOG consecutive leaves starting at `first`.
-template <uint32_t KIND, uint32_t NC, uint32_t LPT_LOG>
-__device__ __forceinline__ void lane_subtree(const LeafSrc& L, uint64_t first, uint32_t out[8]) {
+template <uint32_t KIND, uint32_t NC, uint32_t LPT_LOG, bool WIDE>
+__device__ __forceinline__ void lane_subtree(const LeafSrc& L, uint64_t first, uint32_t (&out)[8]) {
   static_assert(LPT_LOG >= 2 && LPT_LOG <= 4, "lane subtree covers 4..16 leaves");
   constexpr bool kGeneric = KIND == LEAF_COLS && NC == 0;
   constexpr bool kDirect = kGeneric || KIND == LEAF_D2_QUOTIENT || KIND == LEAF_LIFTED ||
@@ -485,13 +518,13 @@ __device__ __forceinline__ void lane_subtree(const LeafSrc& L, uint64_t first, u
     if constexpr (KIND == LEAF_LIFTED_RLC) lifted_rlc_produce(L, i, g);
     if constexpr (KIND == LEAF_CAIRO_QUOTIENT) cairo_readback(L, i, g);
     uint32_t a[8], b[8], n1a[8], n1b[8], n2[8];
-    leaf_hash<KIND, NC>(L, g, gc, i, 0, a);
-    leaf_hash<KIND, NC>(L, g, gc, i, 1, b);
-    b2_hash_node(a, b, n1a);
-    leaf_hash<KIND, NC>(L, g, gc, i, 2, a);
-    leaf_hash<KIND, NC>(L, g, gc, i, 3, b);
-    b2_hash_node(a, b, n1b);
-    b2_hash_node(n1a, n1b, n2);
+    leaf_hash<KIND, NC, WIDE>(L, g, gc, i, 0, a);
+    leaf_hash<KIND, NC, WIDE>(L, g, gc, i, 1, b);
+    hash_node<WIDE>(a, b, n1a);
+    leaf_hash<KIND, NC, WIDE>(L, g, gc, i, 2, a);
+    leaf_hash<KIND, NC, WIDE>(L, g, gc, i, 3, b);
+    hash_node<WIDE>(a, b, n1b);
+    hash_node<WIDE>(n1a, n1b, n2);
     if constexpr (LPT_LOG == 2) {
       cp8(out, n2);
     } else {
@@ -499,12 +532,12 @@ __device__ __forceinline__ void lane_subtree(const LeafSrc& L, uint64_t first, u
         cp8(s2, n2);
       } else {
         uint32_t n3[8];
-        b2_hash_node(s2, n2, n3);
+        hash_node<WIDE>(s2, n2, n3);
         if constexpr (LPT_LOG == 3) {
           cp8(out, n3);
         } else {
           if ((gi & 2) == 0) cp8(s3, n3);
-          else b2_hash_node(s3, n3, out);
+          else hash_node<WIDE>(s3, n3, out);
         }
       }
     }
@@ -514,17 +547,17 @@ __device__ __forceinline__ void lane_subtree(const LeafSrc& L, uint64_t first, u
   }
 }
 
-// One leaf per lane (small, latency-bound trees): the producers work on
+// One leaf per lane (small and middle trees): the producers work on
 // groups of four leaves, so each lane computes the words of its group (the
 // group's four lanes load the same addresses) and hashes leaf idx & 3; only
 // the group's first lane stores produced values (fold layer, quotient).
-template <uint32_t KIND, uint32_t NC>
-__device__ __forceinline__ void lane_leaf(const LeafSrc& L, uint64_t idx, uint32_t out[8]) {
+template <uint32_t KIND, uint32_t NC, bool WIDE>
+__device__ __forceinline__ void lane_leaf(const LeafSrc& L, uint64_t idx, uint32_t (&out)[8]) {
   constexpr bool kGeneric = KIND == LEAF_COLS && NC == 0;
   if constexpr (KIND == LEAF_LIFTED) {
-    lifted_leaf(L, idx, out);
+    lifted_leaf<WIDE>(L, idx, out);
   } else if constexpr (KIND == LEAF_CAIRO_QUOTIENT) {
-    cairo_leaf(L, idx, out);
+    cairo_leaf<WIDE>(L, idx, out);
   } else {
     const uint64_t i = idx & ~3ull;
     const uint32_t j = (uint32_t)idx & 3u;
@@ -539,7 +572,7 @@ __device__ __forceinline__ void lane_leaf(const LeafSrc& L, uint64_t idx, uint32
       uint32_t w[16];
 #pragma unroll
       for (uint32_t c = 0; c < 16; c++) w[c] = pick(gc.c[c].x, gc.c[c].y, gc.c[c].z, gc.c[c].w);
-      b2_hash_words(w, L.n_cols, out);
+      hash_words<WIDE>(w, L.n_cols, out);
       return;
     } else if constexpr (KIND == LEAF_D2_QUOTIENT) {
       d2_produce(L, i, g, first);
@@ -557,12 +590,12 @@ __device__ __forceinline__ void lane_leaf(const LeafSrc& L, uint64_t idx, uint32
       leaf_produce<KIND, NC>(L, i, r, aq, af, am, g, first);
     }
     if constexpr (KIND == LEAF_COLS && NC == 1) {
-      b2_leaf1(pick(g.w[0][0], g.w[1][0], g.w[2][0], g.w[3][0]), out);
+      leaf1<WIDE>(pick(g.w[0][0], g.w[1][0], g.w[2][0], g.w[3][0]), out);
     } else {
       uint32_t w[4];
 #pragma unroll
       for (int c = 0; c < 4; c++) w[c] = pick(g.w[0][c], g.w[1][c], g.w[2][c], g.w[3][c]);
-      b2_leaf4(w[0], w[1], w[2], w[3], out);
+      leaf4<WIDE>(w[0], w[1], w[2], w[3], out);
     }
   }
 }
@@ -693,7 +726,7 @@ __device__ __forceinline__ void lds_merge_in_place(uint32_t* s, uint32_t cnt, ui
         const uint32_t* c = lds_node(s, 2 * tid);
 #pragma unroll
         for (int k = 0; k < 4; k++) u4w(ld4(c + 4 * k), m + 4 * k);
-        b2_hash_node(m, m + 8, node);
+        b2_hash_node_wide(m, m + 8, node);
       }
       __syncthreads();
       if (tid < cnt) {
@@ -709,11 +742,13 @@ __device__ __forceinline__ void lds_merge_in_place(uint32_t* s, uint32_t cnt, ui
 // ROOT instances (the whole tree in one workgroup) carry the transcript step;
 // the throughput instances do not, which keeps their VGPR count (and so their
 // occupancy) at what the hashing itself needs.
-template <uint32_t KIND, uint32_t NC, uint32_t LPT_LOG, bool ROOT>
+// WIDE (at least two wavefronts per SIMD) hashes by b2_compress_wide and
+// merges in place.
+template <uint32_t KIND, uint32_t NC, uint32_t LPT_LOG, bool ROOT, bool WIDE>
 __global__ __launch_bounds__(SUB_THREADS) void k_subtree(LeafSrc L, TreeLevels T, uint32_t tile_log,
                                                          uint32_t store_lo, RootHook hook) {
-  constexpr bool IN_PLACE = !ROOT && LPT_LOG >= 2;
-  __shared__ uint4 buf[IN_PLACE ? 1 : 2][IN_PLACE ? lds_nodes(SUB_THREADS) / 4 : 2 * SUB_THREADS];
+  static_assert(!(ROOT && WIDE), "the transcript step follows the latency-bound merge");
+  __shared__ uint4 buf[WIDE ? 1 : 2][WIDE ? lds_nodes(SUB_THREADS) / 4 : 2 * SUB_THREADS];
   const uint32_t nthr = 1u << (tile_log - LPT_LOG);
   const uint32_t tid = threadIdx.x;
   const uint64_t tile = blockIdx.x;
@@ -735,15 +770,15 @@ __global__ __launch_bounds__(SUB_THREADS) void k_subtree(LeafSrc L, TreeLevels T
   }
   if (tid < nthr) {
     const uint64_t first = (tile << tile_log) + ((uint64_t)tid << LPT_LOG);
-    if constexpr (LPT_LOG == 0) lane_leaf<KIND, NC>(L, first, node);
-    else lane_subtree<KIND, NC, LPT_LOG>(L, first, node);
-    if constexpr (IN_PLACE) store_node(lds_node(reinterpret_cast<uint32_t*>(buf), tid), node);
+    if constexpr (LPT_LOG == 0) lane_leaf<KIND, NC, WIDE>(L, first, node);
+    else lane_subtree<KIND, NC, LPT_LOG, WIDE>(L, first, node);
+    if constexpr (WIDE) store_node(lds_node(reinterpret_cast<uint32_t*>(buf), tid), node);
     else lds_put(buf[0], tid, node);
     if (T.base && LPT_LOG >= store_lo)
       store_node(T.base + T.off[LPT_LOG] + 8 * ((tile << (tile_log - LPT_LOG)) + tid), node);
   }
   __syncthreads();
-  if constexpr (IN_PLACE)
+  if constexpr (WIDE)
     lds_merge_in_place(reinterpret_cast<uint32_t*>(buf), nthr, LPT_LOG, T, tile, tile_log, store_lo);
   else
     lds_merge<SUB_THREADS>(buf, nthr, LPT_LOG, T, tile, tile_log, store_lo, node);
@@ -803,15 +838,24 @@ static uint32_t lane_log_for(uint32_t tile_log) {
   return l < 2 ? 2 : (l > 4 ? 4 : l);
 }
 
+// Two wavefronts per SIMD (512 workgroups of 256 lanes on 256 CUs) is where
+// b2_compress_wide overtakes b2_compress: 33 -> 40 giga-compressions/s there,
+// 31 -> 24 with one. Shapes of 8 and 16 leaves per lane are for trees whose
+// grids are larger, so they have only that form.
+static bool wide_grid(uint64_t workgroups) { return workgroups >= 512; }
+
 template <uint32_t KIND, uint32_t NC, uint32_t LPT>
 static void launch_subtree_lpt(const LeafSrc& L, const TreeLevels& T, uint32_t tile_log, uint32_t store_lo,
                                const RootHook& hook, hipStream_t s) {
   const uint64_t grid = 1ull << (T.log_n - tile_log);
   if (tile_log == T.log_n)
-    hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, true>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
+    hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, true, false>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
+                       tile_log, store_lo, hook);
+  else if (LPT >= 3 || wide_grid(grid))
+    hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, false, true>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
                        tile_log, store_lo, hook);
   else
-    hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, false>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
+    hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, false, LPT >= 3>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
                        tile_log, store_lo, hook);
 }
 
@@ -1087,6 +1131,7 @@ void fri_tail(const FriTailArgs& a, hipStream_t s) {
 }
 
 // ------------------------------------------------------- reference-API kernels
+template <bool WIDE>
 __global__ void k_leaf_hashes(LeafSrc L, uint64_t n, uint32_t* hashes) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -1094,16 +1139,19 @@ __global__ void k_leaf_hashes(LeafSrc L, uint64_t n, uint32_t* hashes) {
   uint32_t nc = L.n_cols > 16 ? 16 : L.n_cols;
   for (uint32_t c = 0; c < 16; c++) w[c] = c < nc ? L.col[c][i] : 0u;
   uint32_t h[8];
-  b2_hash_words(w, nc, h);
+  if constexpr (WIDE) b2_hash_words_wide(w, nc, h);
+  else b2_hash_words(w, nc, h);
   store_node(hashes + 8 * i, h);
 }
 void merkle_leaf_hashes(const LeafSrc& L, uint64_t n, uint32_t* hashes, hipStream_t s) {
   require(L.kind == LEAF_COLS && L.n_cols >= 1 && L.n_cols <= 16, "merkle_hash_leaves: 1..16 columns");
   if (n == 0) return;
-  hipLaunchKernelGGL(k_leaf_hashes, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, L, n, hashes);
+  hipLaunchKernelGGL(wide_grid(n / 256) ? k_leaf_hashes<true> : k_leaf_hashes<false>, dim3((uint32_t)((n + 255) / 256)),
+                     dim3(256), 0, s, L, n, hashes);
   VX_HIP(hipGetLastError());
 }
 
+template <bool WIDE>
 __global__ void k_hash_nodes(const uint32_t* ch, uint32_t* par, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -1112,12 +1160,14 @@ __global__ void k_hash_nodes(const uint32_t* ch, uint32_t* par, uint64_t n) {
     l[k] = ch[16 * i + k];
     r[k] = ch[16 * i + 8 + k];
   }
-  b2_hash_node(l, r, h);
+  if constexpr (WIDE) b2_hash_node_wide(l, r, h);
+  else b2_hash_node(l, r, h);
   store_node(par + 8 * i, h);
 }
 void merkle_hash_nodes(const uint32_t* children, uint32_t* parents, uint64_t n, hipStream_t s) {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_hash_nodes, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, children, parents, n);
+  hipLaunchKernelGGL(wide_grid(n / 256) ? k_hash_nodes<true> : k_hash_nodes<false>, dim3((uint32_t)((n + 255) / 256)),
+                     dim3(256), 0, s, children, parents, n);
   VX_HIP(hipGetLastError());
 }
 
@@ -1193,17 +1243,19 @@ void merkle_leaf_pairs(const LeafSrc& L, uint64_t n_leaves, uint32_t* parents, h
   VX_HIP(hipGetLastError());
 }
 
+template <bool WIDE>
 __global__ void k_lifted_leaves(LeafSrc L, uint64_t n, uint32_t* hashes) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   uint32_t h[8];
-  lifted_leaf(L, i, h);
+  lifted_leaf<WIDE>(L, i, h);
   store_node(hashes + 8 * i, h);
 }
 void merkle_lifted_leaves(const LeafSrc& L, uint32_t* hashes, hipStream_t s) {
   check_leaf(L, L.lift_log);
   const uint64_t n = 1ull << L.lift_log;
-  hipLaunchKernelGGL(k_lifted_leaves, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, L, n, hashes);
+  hipLaunchKernelGGL(wide_grid(n / 256) ? k_lifted_leaves<true> : k_lifted_leaves<false>, dim3((uint32_t)((n + 255) / 256)),
+                     dim3(256), 0, s, L, n, hashes);
   VX_HIP(hipGetLastError());
 }
 
@@ -1267,7 +1319,7 @@ __global__ __launch_bounds__(64) void k_decommit(const DecomDesc* descs, const u
   if (lane < (1u << lo)) {
     uint32_t h[8];
     if (d.kind == DECOM_LIFTED) {
-      lifted_leaf_cols(d.lift, d.n_cols, D, first + lane, h);
+      lifted_leaf_cols<false>(d.lift, d.n_cols, D, first + lane, h);
     } else {
       uint32_t w[16];
       decom_value(d, first + lane, w);

@@ -100,19 +100,12 @@ VX_HD void ch_pow_prefix(const Channel& c, uint32_t pow_bits, uint32_t out[8]) {
   b2_compress(out, m, 52u, true);
 }
 
-// Trailing zeros of the first 16 bytes (u128 LE) of Blake2s(prefix || nonce).
-// With M31_OUT every output word is first reduced mod P, as stwo's
+// Trailing zeros of the first 16 bytes (u128 LE) of a Blake2s digest. With
+// M31_OUT every output word is first reduced mod P, as stwo's
 // Blake2sChannelGeneric<true> hashes (cuda/grind_m31_output.cu:44-63): a
 // 32-bit word x becomes (x & P) + (x >> 31), less P when that reaches P.
 template <bool M31_OUT = false>
-VX_HD uint32_t pow_trailing_zeros(const uint32_t prefix[8], uint64_t nonce) {
-  uint32_t m[16] = {0};
-  for (int i = 0; i < 8; i++) m[i] = prefix[i];
-  m[8] = (uint32_t)nonce;
-  m[9] = (uint32_t)(nonce >> 32);
-  uint32_t h[8];
-  b2_init(h);
-  b2_compress(h, m, 40u, true);
+VX_HD uint32_t digest_trailing_zeros(const uint32_t h[4]) {
   for (int i = 0; i < 4; i++) {
     uint32_t w = h[i];
     if (M31_OUT) {
@@ -122,6 +115,19 @@ VX_HD uint32_t pow_trailing_zeros(const uint32_t prefix[8], uint64_t nonce) {
     if (w) return 32u * i + (uint32_t)__builtin_ctz(w);
   }
   return 128u;
+}
+
+// The same of Blake2s(prefix || nonce).
+template <bool M31_OUT = false>
+VX_HD uint32_t pow_trailing_zeros(const uint32_t prefix[8], uint64_t nonce) {
+  uint32_t m[16] = {0};
+  for (int i = 0; i < 8; i++) m[i] = prefix[i];
+  m[8] = (uint32_t)nonce;
+  m[9] = (uint32_t)(nonce >> 32);
+  uint32_t h[8];
+  b2_init(h);
+  b2_compress(h, m, 40u, true);
+  return digest_trailing_zeros<M31_OUT>(h);
 }
 
 }  // namespace vx
