@@ -42,6 +42,8 @@ static constexpr uint32_t RED_THREADS = 512;  // tree-top reduce: 1024 nodes, 10
 static constexpr uint32_t RED_NLEV_MAX = 10;
 static constexpr uint32_t RED_QUAD_NLEV = 8;  // 4 x 2^(8-1) lanes: the first level by quads
 static constexpr uint32_t TAIL_THREADS = 1u << TAIL_MAX_LOG;  // one lane per leaf of the largest tail layer
+static constexpr uint32_t TAIL_QUAD_LEAVES = 128;  // at most: leaves hashed by quads (two wavefronts per SIMD)
+static constexpr uint32_t TAIL_WIDE = 512;         // from here: two wavefronts per SIMD with one leaf per lane
 
 struct G4 {
   uint32_t w[4][4];  // words of 4 consecutive leaves (W <= 4)
@@ -636,6 +638,14 @@ __device__ __forceinline__ void finish_root_q0(const RootHook& h, const uint32_t
   }
 }
 
+// Where the first stored level above lvl0 begins (null when none is stored).
+// The levels lie back to back, so a merge steps from one to the next: their
+// offsets in the kernel's arguments would be a scalar load per level, waited
+// for on the chain of hashes.
+__device__ __forceinline__ uint32_t* first_stored(const TreeLevels& T, uint32_t lvl0, uint32_t store_lo) {
+  return T.base ? T.base + T.off[lvl0 + 1 > store_lo ? lvl0 + 1 : store_lo] : nullptr;
+}
+
 // Merges `nthr` nodes held one per lane in `buf[0]` up to one node, storing
 // each produced level (lvl0+1 ...) at global index base_idx(level) + lane.
 // Returns the top node in lane 0's `node`.
@@ -650,8 +660,10 @@ __device__ __forceinline__ void lds_merge(uint4 (*buf)[2 * CAP], uint32_t nthr, 
   const uint32_t tid = threadIdx.x;
   uint32_t cur = 0;
   uint32_t cnt = nthr;
+  uint32_t* g = first_stored(T, lvl0, store_lo);
   for (uint32_t lvl = lvl0 + 1; cnt > 1; lvl++) {
     cnt >>= 1;
+    const bool store = g && lvl >= store_lo;
     if (4 * cnt <= CAP) {
       const uint32_t nid = tid >> 2, q = tid & 3;
       if (nid < cnt) {
@@ -664,10 +676,10 @@ __device__ __forceinline__ void lds_merge(uint4 (*buf)[2 * CAP], uint32_t nthr, 
         uint32_t* dst = reinterpret_cast<uint32_t*>(buf[cur ^ 1]) + 8 * nid;
         dst[q] = lo;
         dst[4 + q] = hi;
-        if (T.base && lvl >= store_lo) {
-          uint32_t* g = T.base + T.off[lvl] + 8 * ((group << (group_log - lvl)) + nid);
-          g[q] = lo;
-          g[4 + q] = hi;
+        if (store) {
+          uint32_t* o = g + 8 * ((group << (group_log - lvl)) + nid);
+          o[q] = lo;
+          o[4 + q] = hi;
         }
       }
     } else if (tid < cnt) {
@@ -676,9 +688,9 @@ __device__ __forceinline__ void lds_merge(uint4 (*buf)[2 * CAP], uint32_t nthr, 
       lds_get(buf[cur], 2 * tid + 1, r);
       b2_hash_node(l, r, node);
       lds_put(buf[cur ^ 1], tid, node);
-      if (T.base && lvl >= store_lo)
-        store_node(T.base + T.off[lvl] + 8 * ((group << (group_log - lvl)) + tid), node);
+      if (store) store_node(g + 8 * ((group << (group_log - lvl)) + tid), node);
     }
+    if (store) g += 8ull << (T.log_n - lvl);
     cur ^= 1;
     __syncthreads();
   }
@@ -698,14 +710,16 @@ __device__ __forceinline__ void lds_merge_in_place(uint32_t* s, uint32_t cnt, ui
                                                    uint64_t group, uint32_t group_log, uint32_t store_lo) {
   const uint32_t tid = threadIdx.x, nid = tid >> 2, q = tid & 3;
   const QuadOff o = quad_off(quad_row(q), 4 * QUAD_STRIDE * nid);
+  uint32_t* level = first_stored(T, lvl, store_lo);
   while (cnt > 1) {
     cnt >>= 1;
     lvl++;
     // levels of at most 16 nodes are the first wavefront's: no barrier
     const bool solo = cnt <= 16;
     if (solo && tid >= 64) return;
-    const bool store = T.base && lvl >= store_lo;
-    uint32_t* g = store ? T.base + T.off[lvl] + 8 * (group << (group_log - lvl)) : nullptr;
+    const bool store = level && lvl >= store_lo;
+    uint32_t* g = level + 8 * (group << (group_log - lvl));
+    if (store) level += 8ull << (T.log_n - lvl);
     if (4 * cnt <= SUB_THREADS) {
       uint32_t lo = 0, hi = 0;
       if (nid < cnt) b2_hash_x4_lds(s, o, 64u, q, lo, hi);
@@ -980,6 +994,8 @@ void merkle_commit_shaped(const LeafSrc& L, const TreeLevels& T, uint32_t store_
           "merkle_commit: invalid tree shape");
   require(store_lo >= T.lo && store_lo >= lpt && store_lo <= tile_log,
           "merkle_commit: stored levels must start at or above the lane level");
+  for (uint32_t l = T.lo; l < T.log_n; l++)
+    require(T.off[l + 1] == T.off[l] + (8ull << (T.log_n - l)), "merkle_commit: tree levels must lie back to back");
   if (sub_begin) VX_HIP(hipEventRecord(sub_begin, s));
   dispatch_subtree(L, T, tile_log, lpt, store_lo, hook, s);
   if (sub_end) VX_HIP(hipEventRecord(sub_end, s));
@@ -1019,23 +1035,35 @@ void merkle_tiled(const LeafSrc& L, uint32_t log_n, uint32_t tile_log, uint32_t*
 // ------------------------------------------------------------ FRI tail
 // FRI line-fold layers of at most 2^TAIL_MAX_LOG values, committed one after
 // another by a single 1024-lane workgroup: fold (previous layer from LDS),
-// one leaf hash per lane, tree levels in LDS (quad hashes once at most 256
-// parents are left; levels >= lo stored for the decommitment), root into the
-// proof, then the quad of lanes 0..3 mixes the root and draws the next alpha
-// (src/prover.rs:527-544). A layer of 2^L values is a dependent chain of
-// two one-lane hashes, L - 1 quad hashes and the two quad channel hashes.
+// leaf hashes, tree levels in LDS (levels >= lo stored for the decommitment),
+// root into the proof, then the quad of lanes 0..3 mixes the root and draws
+// the next alpha (src/prover.rs:527-544).
+//
+// Bound by the dependent chain of hashes. Where a level fills the workgroup's
+// four wavefronts per SIMD it is hashed one node per lane (512 and more by
+// b2_compress_wide), from 256 nodes down (leaves: 128) by quads. Levels of at
+// most 16 nodes belong to the first wavefront and need no barrier. Nothing on
+// the chain waits for HBM: the channel stays in registers, the challenge in
+// LDS, and a layer's twiddles are loaded while the layer before is hashed.
+// Eight layers from 2^10 values: 97 -> 90 us.
 __global__ __launch_bounds__(TAIL_THREADS) void k_fri_tail(FriTailArgs a) {
   __shared__ uint32_t vals[2][4][1u << TAIL_MAX_LOG];
   __shared__ uint4 hashes[2u << TAIL_MAX_LOG];
   __shared__ uint32_t s_alpha[4];
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x, nid = tid >> 2, q = tid & 3;
+  uint32_t* const words = reinterpret_cast<uint32_t*>(hashes);
+  Channel ch{};
+  if (tid < 4) {
+    ch = *a.ch;
+    s_alpha[q] = a.layer[0].alpha[q];
+  }
+  uint32_t tw = tid < (1u << a.layer[0].log_n) ? a.layer[0].tw[tid] : 0u;
   uint32_t cur = 0;
   for (uint32_t li = 0; li < a.n_layers; li++) {
     const FriTailLayer& T = a.layer[li];
     const uint32_t L = T.log_n, n = 1u << L;
-    if (tid == 0)
-      for (int k = 0; k < 4; k++) s_alpha[k] = T.alpha[k];
-    __syncthreads();
+    const bool quad_leaves = n <= TAIL_QUAD_LEAVES;
+    __syncthreads();  // the challenge is drawn, the last layer's nodes are done with
     const qm31_mat am = qm_left_matrix(qm31{{s_alpha[0], s_alpha[1], s_alpha[2], s_alpha[3]}});
     if (tid < n) {
       const uint32_t i = tid;
@@ -1048,37 +1076,50 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_fri_tail(FriTailArgs a) {
         f0 = {{vals[p][0][2 * i], vals[p][1][2 * i], vals[p][2][2 * i], vals[p][3][2 * i]}};
         f1 = {{vals[p][0][2 * i + 1], vals[p][1][2 * i + 1], vals[p][2][2 * i + 1], vals[p][3][2 * i + 1]}};
       }
-      const qm31 r = fri_fold_pair_m(f0, f1, am, T.tw[i]);
+      const qm31 r = fri_fold_pair_m(f0, f1, am, tw);
       for (int c = 0; c < 4; c++) {
         vals[cur][c][i] = r.v[c];
         T.out[c][i] = r.v[c];
       }
-      uint32_t h[8];
-      b2_leaf4(r.v[0], r.v[1], r.v[2], r.v[3], h);
-      lds_put(hashes, i, h);
+      if (!quad_leaves) {
+        uint32_t h[8];
+        if (n >= TAIL_WIDE) leaf4<true>(r.v[0], r.v[1], r.v[2], r.v[3], h);
+        else leaf4<false>(r.v[0], r.v[1], r.v[2], r.v[3], h);
+        lds_put(hashes, i, h);
+      }
     }
+    if (li + 1 < a.n_layers) tw = tid < n / 2 ? a.layer[li + 1].tw[tid] : 0u;
     __syncthreads();
+    if (quad_leaves) {
+      if (nid < n) {
+        const uint32_t m[16] = {vals[cur][0][nid], vals[cur][1][nid], vals[cur][2][nid], vals[cur][3][nid]};
+        uint32_t lo, hi;
+        b2_hash_x4(m, 16u, q, lo, hi);
+        words[8 * nid + q] = lo;
+        words[8 * nid + 4 + q] = hi;
+      }
+      __syncthreads();
+    }
+    uint32_t* level = T.tree + T.off[T.lo];  // the stored levels lie back to back
     for (uint32_t lvl = 1; lvl <= L; lvl++) {
       const uint32_t cnt = n >> lvl;
+      const bool solo = cnt <= 16, store = lvl >= T.lo;
+      if (solo && tid >= 64) break;
       if (4 * cnt <= TAIL_THREADS) {
-        const uint32_t nid = tid >> 2, q = tid & 3;
         uint32_t lo = 0, hi = 0;
         if (nid < cnt) {
-          const uint32_t* src = reinterpret_cast<const uint32_t*>(hashes) + 16 * nid;
           uint32_t m[16];
 #pragma unroll
-          for (int k = 0; k < 16; k++) m[k] = src[k];
+          for (int k = 0; k < 16; k++) m[k] = words[16 * nid + k];
           b2_node_x4(m, q, lo, hi);
         }
-        __syncthreads();  // every child read before any parent overwrites it
+        if (!solo) __syncthreads();  // every child read before any parent overwrites it
         if (nid < cnt) {
-          uint32_t* dst = reinterpret_cast<uint32_t*>(hashes) + 8 * nid;
-          dst[q] = lo;
-          dst[4 + q] = hi;
-          if (lvl >= T.lo) {
-            uint32_t* g = T.tree + T.off[lvl] + 8 * nid;
-            g[q] = lo;
-            g[4 + q] = hi;
+          words[8 * nid + q] = lo;
+          words[8 * nid + 4 + q] = hi;
+          if (store) {
+            level[8 * nid + q] = lo;
+            level[8 * nid + 4 + q] = hi;
           }
         }
       } else {
@@ -1086,31 +1127,34 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_fri_tail(FriTailArgs a) {
         if (tid < cnt) {
           lds_get(hashes, 2 * tid, l);
           lds_get(hashes, 2 * tid + 1, r);
-          b2_hash_node(l, r, p);
+          hash_node<true>(l, r, p);
         }
         __syncthreads();
         if (tid < cnt) {
           lds_put(hashes, tid, p);
-          if (lvl >= T.lo) store_node(T.tree + T.off[lvl] + 8 * tid, p);
+          if (store) store_node(level + 8 * tid, p);
         }
       }
-      __syncthreads();
+      if (store) level += 8 * cnt;
+      if (solo) wave_lds_order();
+      else __syncthreads();
     }
     if (tid < 4) {
       uint32_t root[8];
       lds_get(hashes, 0, root);
       if (tid == 0)
         for (int k = 0; k < 8; k++) T.root_out[k] = root[k];
-      Channel c = *a.ch;
-      ch_mix_digest_q0(c, root, tid);
+      ch_mix_digest_q0(ch, root, tid);
       if (T.next_alpha) {
-        const qm31 nx = ch_draw_felt_q0(c, tid);
+        const qm31 nx = ch_draw_felt_q0(ch, tid);
         if (tid == 0)
-          for (int k = 0; k < 4; k++) T.next_alpha[k] = nx.v[k];
+          for (int k = 0; k < 4; k++) {
+            T.next_alpha[k] = nx.v[k];
+            s_alpha[k] = nx.v[k];
+          }
       }
-      if (tid == 0) *a.ch = c;
+      if (tid == 0 && li + 1 == a.n_layers) *a.ch = ch;
     }
-    __syncthreads();
     cur ^= 1;
   }
 }
@@ -1123,6 +1167,8 @@ void fri_tail(const FriTailArgs& a, hipStream_t s) {
     require(T.log_n >= 1 && T.log_n <= TAIL_MAX_LOG && T.lo <= T.log_n && T.tw && T.tree && T.root_out && T.alpha,
             "fri_tail: bad layer");
     require(li == 0 || T.log_n + 1 == prev, "fri_tail: layers must halve");
+    for (uint32_t l = T.lo; l < T.log_n; l++)
+      require(T.off[l + 1] == T.off[l] + (8u << (T.log_n - l)), "fri_tail: tree levels must lie back to back");
     for (int c = 0; c < 4; c++) require(T.out[c] != nullptr && (li > 0 || a.in[c] != nullptr), "fri_tail: null column");
     prev = T.log_n;
   }
