@@ -6,6 +6,7 @@
 // memory. Query draws are independent squeezes (n_draws = 0..nq-1 after
 // mix_felts), so one lane per query computes them in parallel.
 #include "vx_blake2s_wide.h"
+#include "vx_blake2s_x4.h"
 #include "vx_internal.h"
 
 namespace vx {
@@ -39,22 +40,77 @@ void channel_step(Channel* ch, bool init, const uint32_t* digest, uint32_t* alph
 }
 
 // mix_felts(last layer) (src/prover.rs:554); writes n_last + the 8 values
-// into the proof and, for PoW, the prefix digest of the new state.
-__global__ void k_mix_last(QueryArgs q, uint32_t* prefix_out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  Channel c = *q.ch;
-  uint32_t w[32];
-  for (int i = 0; i < 8; i++)
-    for (int k = 0; k < 4; k++) w[4 * i + k] = q.last[k][i];
-  ch_mix_felts(c, w, 8);
-  q.proof[q.last_word] = 8;
-  for (int i = 0; i < 32; i++) q.proof[q.last_word + 1 + i] = w[i];
-  if (q.pow_bits && prefix_out) ch_pow_prefix(c, q.pow_bits, prefix_out);
-  *q.ch = c;
+// into the proof. With PoW: the prefix digest of the new state, and the search's
+// nonce set to "none". Without: the queries too, when one workgroup's lanes
+// cover them (MIX_QUERIES_MAX), so that the step is one launch.
+//
+// A dependent chain of three or four compressions: by the quad of lanes 0..3 on
+// words in LDS: 6.0 us with the queries, where one lane took 7.7 us and the
+// queries a launch of 4.4 us more.
+static constexpr uint32_t MIX_THREADS = 256, MIX_QUERIES_MAX = MIX_THREADS;
+
+__device__ __forceinline__ void draw_query(const QueryArgs& q, Channel c, uint32_t i) {
+  c.n_draws = i;
+  const uint32_t v = (uint32_t)ch_draw_number(c, q.domain);
+  q.queries[i] = v;
+  q.proof[q.query_word + 1 + i] = v;
 }
-void channel_mix_last(const QueryArgs& q, uint32_t* prefix_out, hipStream_t s) {
-  hipLaunchKernelGGL(k_mix_last, dim3(1), dim3(64), 0, s, q, prefix_out);
-  VX_HIP(hipGetLastError());
+
+__global__ __launch_bounds__(MIX_THREADS) void k_mix_last(QueryArgs q, uint32_t* prefix_out, uint64_t* nonce_out) {
+  __shared__ uint32_t msg[48];  // state || 8 QM31 values, zero-padded to whole blocks
+  __shared__ uint32_t state[8];
+  const uint32_t tid = threadIdx.x;
+  if (tid < 8) {
+    msg[tid] = q.ch->state[tid];
+  } else if (tid < 40) {
+    const uint32_t i = tid - 8, v = q.last[i & 3][i >> 2];
+    msg[tid] = v;
+    q.proof[q.last_word + 1 + i] = v;
+  } else if (tid < 48) {
+    msg[tid] = 0;
+  } else if (tid == 48) {
+    q.proof[q.last_word] = 8;
+    if (!q.pow_bits) q.proof[q.query_word] = q.nq;
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const uint32_t l = tid & 3;
+    const bool q0 = l & 1, q1 = l & 2;
+    uint32_t lo = sel4(q0, q1, VX_B2_H0, VX_B2_IV1, VX_B2_IV2, VX_B2_IV3);
+    uint32_t hi = sel4(q0, q1, VX_B2_IV4, VX_B2_IV5, VX_B2_IV6, VX_B2_IV7);
+    uint32_t m[16];
+    for (uint32_t blk = 0; blk < 3; blk++) {
+#pragma unroll
+      for (int k = 0; k < 16; k++) m[k] = msg[16 * blk + k];
+      b2_compress_x4(lo, hi, m, blk < 2 ? 64 * (blk + 1) : 160u, blk == 2, l);
+    }
+    if (tid < 4) {
+      state[l] = lo;
+      state[4 + l] = hi;
+      q.ch->state[l] = lo;
+      q.ch->state[4 + l] = hi;
+    }
+    if (tid == 0) q.ch->n_draws = 0;
+    if (q.pow_bits && prefix_out) {  // ch_pow_prefix
+      wave_lds_order();
+#pragma unroll
+      for (int k = 0; k < 16; k++) m[k] = k == 0 ? 0x12345678u : k == 12 ? q.pow_bits : k >= 4 && k < 12 ? state[k - 4] : 0u;
+      b2_hash_x4(m, 52u, l, lo, hi);
+      if (tid < 4) {
+        prefix_out[l] = lo;
+        prefix_out[4 + l] = hi;
+      }
+      if (tid == 0) *nonce_out = ~0ull;
+    }
+  }
+  if (q.pow_bits || q.nq > MIX_QUERIES_MAX) return;
+  __syncthreads();
+  if (tid < q.nq) {
+    Channel c;
+#pragma unroll
+    for (int k = 0; k < 8; k++) c.state[k] = state[k];
+    draw_query(q, c, tid);
+  }
 }
 
 // Query i is draw_number(domain) at n_draws = i (src/prover.rs:555-557),
@@ -71,16 +127,16 @@ __global__ void k_draw_queries(QueryArgs q) {
     }
   }
   if (i == 0) q.proof[q.query_word] = q.nq;
-  if (i >= q.nq) return;
-  c.n_draws = i;
-  uint32_t v = (uint32_t)ch_draw_number(c, q.domain);
-  q.queries[i] = v;
-  q.proof[q.query_word + 1 + i] = v;
+  if (i < q.nq) draw_query(q, c, i);
 }
-void channel_draw_queries(const QueryArgs& q, hipStream_t s) {
+
+void channel_queries(const QueryArgs& q, uint32_t* prefix, uint64_t* nonce, hipStream_t s) {
   require(q.nq >= 1 && q.nq <= 65536, "queries: 1..65536 queries");
-  uint32_t blocks = (q.nq + 255) / 256;
-  hipLaunchKernelGGL(k_draw_queries, dim3(blocks), dim3(256), 0, s, q);
+  hipLaunchKernelGGL(k_mix_last, dim3(1), dim3(MIX_THREADS), 0, s, q, prefix, nonce);
+  VX_HIP(hipGetLastError());
+  if (q.pow_bits) grind_pow(prefix, q.pow_bits, nonce, s, true);
+  if (!q.pow_bits && q.nq <= MIX_QUERIES_MAX) return;
+  hipLaunchKernelGGL(k_draw_queries, dim3((q.nq + 255) / 256), dim3(256), 0, s, q);
   VX_HIP(hipGetLastError());
 }
 
@@ -195,10 +251,11 @@ void grind_pow_stwo(const uint32_t* d_prefix, uint32_t pow_bits, uint64_t* d_res
   VX_HIP(hipGetLastError());
 }
 
-void grind_pow(const uint32_t* d_prefix, uint32_t pow_bits, uint64_t* d_result, hipStream_t s) {
+// `preset`: *d_result is ~0 already.
+void grind_pow(const uint32_t* d_prefix, uint32_t pow_bits, uint64_t* d_result, hipStream_t s, bool preset) {
   require(pow_bits >= 1 && pow_bits <= 32, "grind_pow: pow_bits must be 1..32");
   auto* best = reinterpret_cast<unsigned long long*>(d_result);
-  hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(64), 0, s, best, ~0ull);
+  if (!preset) hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(64), 0, s, best, ~0ull);
   // every lane loops until its nonce exceeds the best hit
   launch_grind<false>(grind_grid(pow_bits), false, d_prefix, pow_bits, best, 0ull, GRIND_LIMIT, s);
 }
@@ -214,33 +271,14 @@ void grind_pow_batch(const uint32_t* d_prefix, uint64_t* d_result, uint32_t pow_
   launch_grind<false>(grid, m31_out, d_prefix, pow_bits, best, batch_offset, n, s);
 }
 
-struct WordWrites {
-  uint32_t n;
-  uint32_t off[16];
-  uint32_t val[16];
-};
-__global__ void k_write_words(uint32_t* dst, WordWrites w) {
-  uint32_t i = threadIdx.x;
-  if (i < w.n) dst[w.off[i]] = w.val[i];
-}
-void write_header(uint32_t* proof, const uint32_t* words, uint32_t n, hipStream_t s) {
-  // words: n (offset, value) pairs
-  require(n <= 16, "write_header: at most 16 words");
-  WordWrites w{};
-  w.n = n;
-  for (uint32_t i = 0; i < n; i++) {
-    w.off[i] = words[2 * i];
-    w.val[i] = words[2 * i + 1];
-  }
-  hipLaunchKernelGGL(k_write_words, dim3(1), dim3(64), 0, s, proof, w);
-  VX_HIP(hipGetLastError());
-}
-
 // Proof download by the GPU itself: the workgroups store the proof
 // straight into pinned host memory (mapped into the device's address space),
 // 16 bytes per lane per step, instead of a DMA copy whose start-up cost
 // dominated for 1-2 MB proofs.
-__global__ __launch_bounds__(256) void k_copy_to_host(uint32_t* dst, const uint32_t* src, uint64_t words) {
+// The destination is read from device memory (set_inputs), so that the copy
+// belongs to the proof's captured graph.
+__global__ __launch_bounds__(256) void k_copy_to_host(uint32_t* const* dst_p, const uint32_t* src, uint64_t words) {
+  uint32_t* const dst = *dst_p;
   const uint64_t n16 = words >> 2;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   uint4* d4 = reinterpret_cast<uint4*>(dst);
@@ -250,12 +288,11 @@ __global__ __launch_bounds__(256) void k_copy_to_host(uint32_t* dst, const uint3
   if (tail < (words & 3)) dst[4 * n16 + tail] = src[4 * n16 + tail];
 }
 
-void copy_to_host(uint32_t* host_dst, const uint32_t* dev_src, uint64_t words, hipStream_t s) {
-  require((reinterpret_cast<uintptr_t>(host_dst) & 15u) == 0 && (reinterpret_cast<uintptr_t>(dev_src) & 15u) == 0,
-          "copy_to_host: 16-byte aligned buffers");
+void copy_to_host(uint32_t* const* d_dst, const uint32_t* dev_src, uint64_t words, hipStream_t s) {
+  require((reinterpret_cast<uintptr_t>(dev_src) & 15u) == 0, "copy_to_host: 16-byte aligned buffers");
   const uint64_t blocks = ((words >> 2) + 255) / 256;
   const uint32_t grid = (uint32_t)(blocks < 1 ? 1 : (blocks > 512 ? 512 : blocks));
-  hipLaunchKernelGGL(k_copy_to_host, dim3(grid), dim3(256), 0, s, host_dst, dev_src, words);
+  hipLaunchKernelGGL(k_copy_to_host, dim3(grid), dim3(256), 0, s, d_dst, dev_src, words);
   VX_HIP(hipGetLastError());
 }
 

@@ -78,18 +78,22 @@ void fib_trace_dev(const uint32_t* ab, uint32_t* out, uint32_t log_n, hipStream_
 }
 
 // inputs[0..1] = (a, b) and the proof header words that carry them
-// (Fibonacci: the public inputs; multi-column AIR: the trace seed words).
-__global__ void k_set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b) {
+// (Fibonacci: the public inputs; multi-column AIR: the trace seed words);
+// inputs[2..3] = where the finished proof is copied to.
+__global__ void k_set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b,
+                             uint32_t* host_dst) {
   if (threadIdx.x == 0) {
     inputs[0] = a;
     inputs[1] = b;
+    *reinterpret_cast<uint32_t**>(inputs + 2) = host_dst;
     proof[word_a] = a;
     proof[word_a + 1] = b;
   }
 }
 
-void set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b, hipStream_t s) {
-  hipLaunchKernelGGL(k_set_inputs, dim3(1), dim3(64), 0, s, inputs, proof, word_a, a, b);
+void set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b, uint32_t* host_dst,
+                hipStream_t s) {
+  hipLaunchKernelGGL(k_set_inputs, dim3(1), dim3(64), 0, s, inputs, proof, word_a, a, b, host_dst);
   VX_HIP(hipGetLastError());
 }
 

@@ -304,7 +304,25 @@ StarkProver::StarkProver(uint32_t log_n, uint32_t blowup_bits, uint32_t n_querie
   for (auto& e : ev_) VX_HIP(hipEventCreate(&e));
   tab_ = ProverTables::get(log_n_, blowup_, stream_);
   if (batch) build_batch();
+  else write_header();
   build_descs();
+}
+
+// The proof words that every proof of this prover has alike.
+void StarkProver::write_header() {
+  const ProofLayout& L = layout_;
+  auto put = [&](uint64_t word, const std::vector<uint32_t>& v) {
+    VX_HIP(hipMemcpy(proof_.u32() + word, v.data(), 4 * v.size(), hipMemcpyHostToDevice));
+  };
+  if (air_.kind == AIR_FIBONACCI) {  // words 3, 4 (a, b) are written by set_inputs
+    put(0, {KRAK_MAGIC, pow_bits_ ? 2u : 1u, log_n_});
+    if (pow_bits_) put(5, {blowup_, pow_bits_});
+  } else {  // words 9, 10 (seed) by set_inputs, 7, 8 (nonce) by the query step or 0
+    put(0, {KRAK_MAGIC, 3, log_n_, air_.n_cols, air_.n_cons, blowup_, pow_bits_, 0, 0});
+    put(11, {(uint32_t)air_.air_seed, (uint32_t)(air_.air_seed >> 32), n_groups_});
+  }
+  put(L.w_nfri, {n_fri_});
+  put(L.w_nfdec, {n_fri_});
 }
 
 // Work lists, lifted column table, column offsets and the constant header
@@ -480,20 +498,6 @@ void StarkProver::record(bool timed, hipStream_t s) {
     merkle_commit(lq, tree_levels(QT), tree_lo_[QT], RootHook{d_channel_, proof + L.w_qroot, alpha(1), 0}, s);
     mark(5);
   }
-  std::vector<uint32_t> hw;
-  if (batch) {
-  } else if (!d2) {  // words 3, 4 (a, b) are written by set_inputs
-    hw = {0, KRAK_MAGIC, 1, pow_bits_ ? 2u : 1u, 2, log_n_};
-    if (pow_bits_) hw.insert(hw.end(), {5, blowup_, 6, pow_bits_});
-  } else {    // words 9, 10 (seed) by set_inputs, 7, 8 (nonce) by the query step or stay 0
-    hw = {0, KRAK_MAGIC, 1, 3, 2, log_n_, 3, air_.n_cols, 4, air_.n_cons, 5, blowup_, 6, pow_bits_,
-          11, (uint32_t)air_.air_seed, 12, (uint32_t)(air_.air_seed >> 32), 13, G};
-    if (!pow_bits_) hw.insert(hw.end(), {7, 0, 8, 0});
-  }
-  if (!batch) {
-    hw.insert(hw.end(), {(uint32_t)L.w_nfri, n_fri_, (uint32_t)L.w_nfdec, n_fri_});
-    write_header(proof, hw.data(), (uint32_t)hw.size() / 2, s);
-  }
   if (batch) {
   } else if (!d2) {
     fib_trace_dev(d_inputs_, trace_.u32(), log_n_, s);
@@ -612,12 +616,12 @@ void StarkProver::record(bool timed, hipStream_t s) {
   q.last_word = L.w_last;
   q.query_word = L.w_nq;
   q.nonce_word = pow_bits_ ? L.w_nonce : 0;
-  channel_mix_last(q, d_prefix_, s);
-  if (pow_bits_) grind_pow(d_prefix_, pow_bits_, d_nonce_, s);
-  channel_draw_queries(q, s);
+  channel_queries(q, d_prefix_, d_nonce_, s);
   mark(7);
   decommit(reinterpret_cast<const DecomDesc*>(descs_.p), G + 1 + n_fri_, d_queries_, nq_, proof, s);
   mark(8);
+  copy_to_host(reinterpret_cast<uint32_t* const*>(d_inputs_ + 2), proof, layout_.total_words, s);
+  mark(9);
 }
 
 // Captured on a private stream, so work that other threads put on the
@@ -643,9 +647,16 @@ void StarkProver::capture() {
   VX_HIP(e);
 }
 
+// Public inputs and the pinned buffer that takes the proof.
+void StarkProver::put_inputs(uint32_t a, uint32_t b, uint32_t buffer) {
+  const uint32_t word = air_.kind == AIR_D2 ? 9 : air_.kind == AIR_BATCH ? 7 : 3;
+  set_inputs(d_inputs_, proof_.u32(), word, a, b, host_proof_dev_[buffer], stream_);
+}
+
+// Writes into the buffer of the proof that is about to be made.
 void StarkProver::tune() {
   if (tuned_) return;
-  set_inputs(d_inputs_, proof_.u32(), air_.kind == AIR_D2 ? 9 : (air_.kind == AIR_BATCH ? 7 : 3), 1, 1, stream_);
+  put_inputs(1, 1, cur_ ^ 1);
   record(false, stream_);
   VX_HIP(hipStreamSynchronize(stream_));
   tuned_ = true;
@@ -655,21 +666,14 @@ void StarkProver::enqueue(uint32_t a, uint32_t b, bool timed) {
   const bool seeded = air_.kind != AIR_FIBONACCI;  // (a, b) = the trace seed's words
   require(seeded || (a < P && b < P), "prove: public inputs must be canonical M31");
   timed_ = timed;
-  set_inputs(d_inputs_, proof_.u32(), air_.kind == AIR_D2 ? 9 : (air_.kind == AIR_BATCH ? 7 : 3), a, b, stream_);
-  if (timed || !use_graph_) {
-    record(timed, stream_);
-  } else {
-    if (!graph_) {
-      tune();
-      set_inputs(d_inputs_, proof_.u32(), air_.kind == AIR_D2 ? 9 : (air_.kind == AIR_BATCH ? 7 : 3), a, b,
-                 stream_);
-      capture();
-    }
-    VX_HIP(hipGraphLaunch(graph_, stream_));
+  if (!timed && use_graph_ && !graph_) {
+    tune();
+    capture();
   }
+  put_inputs(a, b, cur_ ^ 1);
+  if (timed || !use_graph_) record(timed, stream_);
+  else VX_HIP(hipGraphLaunch(graph_, stream_));
   cur_ ^= 1;
-  copy_to_host(host_proof_dev_[cur_], proof_.u32(), layout_.total_words, stream_);
-  if (timed) VX_HIP(hipEventRecord(ev_[9], stream_));
 }
 
 const uint8_t* StarkProver::wait(size_t* len) {

@@ -108,6 +108,8 @@ class StarkProver {
   }
   // One eager proof of dummy inputs: every merkle_commit of this class is
   // timed by the autotuner (if enabled) before a graph freezes the shapes.
+  void write_header();
+  void put_inputs(uint32_t a, uint32_t b, uint32_t buffer);
   void tune();
   bool graphs() const { return use_graph_; }
   // Device bytes a prover of this class allocates for itself (tables excluded).

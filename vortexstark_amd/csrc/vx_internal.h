@@ -219,7 +219,8 @@ void stwo_twiddles(uint32_t log_n, uint32_t* tw, uint32_t* itw, hipStream_t s);
 // ------------------------------------------------- misc kernels (fri.hip)
 void fib_trace(uint32_t a, uint32_t b, uint32_t* out, uint32_t log_n, hipStream_t s);
 void fib_trace_dev(const uint32_t* ab, uint32_t* out, uint32_t log_n, hipStream_t s);
-void set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b, hipStream_t s);
+void set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b, uint32_t* host_dst,
+                hipStream_t s);
 void fib_quotient(const uint32_t* trace, uint32_t* o0, uint32_t* o1, uint32_t* o2, uint32_t* o3,
                   qm31 alpha, uint64_t offset, uint64_t chunk_n, uint64_t global_n, hipStream_t s);
 void fold_line(const uint32_t* const in[4], const uint32_t* tw, uint32_t* const out[4], qm31 alpha,
@@ -444,11 +445,12 @@ struct QueryArgs {
   uint64_t query_word;      // word offset of n_queries
   uint64_t nonce_word;      // word offset of nonce (v2) or 0
 };
-void channel_mix_last(const QueryArgs& q, uint32_t* prefix_out, hipStream_t s);
-void channel_draw_queries(const QueryArgs& q, hipStream_t s);
+// The transcript from the last FRI layer to the query indices; with PoW the
+// search in between (prefix: 8 words, nonce: device scratch).
+void channel_queries(const QueryArgs& q, uint32_t* prefix, uint64_t* nonce, hipStream_t s);
 // Deterministic PoW: smallest nonce >= 0 (linear order) whose Blake2s has
 // >= pow_bits trailing zeros (src/channel.rs:140-168).
-void grind_pow(const uint32_t* d_prefix, uint32_t pow_bits, uint64_t* d_result, hipStream_t s);
+void grind_pow(const uint32_t* d_prefix, uint32_t pow_bits, uint64_t* d_result, hipStream_t s, bool preset = false);
 // The same search over the stwo plugin's nonces (hi << 32) | low, low < 2^20;
 // m31_out reduces the hash words mod P before the count (stwo's
 // Blake2sChannelGeneric<true>).
@@ -465,10 +467,9 @@ void poseidon_grind_min(const uint64_t* d_prefix_mont, uint32_t pow_bits, uint64
 void poseidon_leaves(const uint32_t* const* d_cols, const uint32_t* d_logs, uint32_t n_cols, uint32_t lifting_log,
                      uint64_t* d_out, uint32_t n_leaves, hipStream_t s);
 void poseidon_next_layer(const uint64_t* d_prev, uint64_t* d_out, uint32_t n_parents, hipStream_t s);
-void write_header(uint32_t* proof, const uint32_t* words, uint32_t n, hipStream_t s);
 // Copy `words` words from device memory into pinned host memory
 // (hipHostMalloc) with a kernel; both 16-byte aligned.
-void copy_to_host(uint32_t* host_dst, const uint32_t* dev_src, uint64_t words, hipStream_t s);
+void copy_to_host(uint32_t* const* d_dst, const uint32_t* dev_src, uint64_t words, hipStream_t s);
 
 // ------------------------------------- synthetic multi-column AIR (d2.hip)
 void d2_trace(const uint32_t* seed_words, uint32_t* out, uint32_t n_cols, uint32_t log_n, uint64_t stride,
