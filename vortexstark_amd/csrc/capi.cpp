@@ -67,6 +67,34 @@ static TwiddleRef tw_ref(const uint32_t* line, const uint32_t* circle, const uin
   return r;
 }
 
+// Runs f(NttCols) over a batch of columns given by host pointer arrays (src may
+// be null). Up to NTT_ARG_COLS columns travel in the kernels' arguments; more
+// are uploaded, in chunks of at most 65535 columns (one grid row each). A
+// table's allocation, pageable upload and free cost about 9 us a call (a
+// commitment of 13 + 27 columns, four such calls and the
+// lifted leaves: 270 us with tables, 225 us without), as much as the launches
+// of one more chunk of NTT_ARG_COLS columns: the line lies there. Returns after
+// the stream has finished, so the table outlives the kernels.
+template <typename F>
+static void ntt_cols(uint32_t* const* dst, const uint32_t* const* src, uint32_t n_cols, hipStream_t s, F&& f) {
+  if (n_cols <= NTT_ARG_COLS) {
+    f(NttCols{dst, src, n_cols, false});
+    VX_HIP(hipStreamSynchronize(s));
+    return;
+  }
+  constexpr uint32_t CHUNK = 65535;
+  const uint32_t m0 = n_cols < CHUNK ? n_cols : CHUNK;
+  DeviceBuf d((src ? 2 : 1) * sizeof(uint32_t*) * (size_t)m0);
+  for (uint32_t c0 = 0; c0 < n_cols; c0 += CHUNK) {
+    const uint32_t m = n_cols - c0 < CHUNK ? n_cols - c0 : CHUNK;
+    uint32_t** dc = static_cast<uint32_t**>(d.p);
+    VX_HIP(hipMemcpyAsync(dc, dst + c0, sizeof(uint32_t*) * m, hipMemcpyHostToDevice, s));
+    if (src) VX_HIP(hipMemcpyAsync(dc + m, src + c0, sizeof(uint32_t*) * m, hipMemcpyHostToDevice, s));
+    f(NttCols{dc, src ? const_cast<const uint32_t* const*>(dc + m) : nullptr, m, true});
+    VX_HIP(hipStreamSynchronize(s));
+  }
+}
+
 extern "C" {
 
 const char* vx_last_error(void) { return g_last_error.c_str(); }
@@ -164,28 +192,19 @@ static std::vector<uint32_t*> fetch_ptrs(const void* arr, uint32_t n, hipStream_
   return h;
 }
 
-// Columns of a batched in-place transform: the host pointer array is checked
-// and copied to the device, in chunks of at most 65535 columns (one grid row
-// each), and every pass runs over a whole chunk in one launch. Returns after
-// the stream has finished, so the staging buffer outlives the kernels.
+// In-place transforms of a batch of columns: the host pointer array is checked.
 static void ntt_cols(uint32_t* const* cols, uint32_t n_cols, const TwiddleRef& r, bool forward, hipStream_t s) {
   if (n_cols == 0) return;
   require(cols != nullptr, "null column array");
   for (uint32_t c = 0; c < n_cols; c++)
     require(cols[c] != nullptr && (reinterpret_cast<uintptr_t>(cols[c]) & 15u) == 0,
             "ntt batch: columns must be non-null and 16-byte aligned");
-  constexpr uint32_t CHUNK = 65535;
-  DeviceBuf d(sizeof(uint32_t*) * (n_cols < CHUNK ? n_cols : CHUNK));
-  for (uint32_t c0 = 0; c0 < n_cols; c0 += CHUNK) {
-    const uint32_t m = n_cols - c0 < CHUNK ? n_cols - c0 : CHUNK;
-    VX_HIP(hipMemcpyAsync(d.p, cols + c0, sizeof(uint32_t*) * m, hipMemcpyHostToDevice, s));
-    uint32_t* const* dc = static_cast<uint32_t* const*>(d.p);
+  ntt_cols(cols, nullptr, n_cols, s, [&](const NttCols& c) {
     if (forward)
-      ntt_forward_cols(dc, m, r, s);
+      ntt_forward_cols(c, r, s);
     else
-      ntt_inverse_cols(dc, m, r, s);
-    VX_HIP(hipStreamSynchronize(s));
-  }
+      ntt_inverse_cols(c, r, s);
+  });
 }
 
 int vx_circle_ntt_evaluate_batch(uint32_t* const* d_cols, const uint32_t* tw, const uint32_t* ctw,
@@ -498,21 +517,8 @@ int vx_stwo_ntt_evaluate_lde_batch(uint32_t* const* h_eval, const uint32_t* cons
       require(((reinterpret_cast<uintptr_t>(h_eval[c]) | reinterpret_cast<uintptr_t>(h_coeffs[c])) & 15u) == 0,
               "stwo lde batch: columns must be 16-byte aligned");
     }
-    constexpr uint32_t CHUNK = 65535;
-    const uint32_t m0 = n_cols < CHUNK ? n_cols : CHUNK;
-    DeviceBuf d(2 * sizeof(uint32_t*) * m0);
-    for (uint32_t c0 = 0; c0 < n_cols; c0 += CHUNK) {
-      const uint32_t m = n_cols - c0 < CHUNK ? n_cols - c0 : CHUNK;
-      std::vector<const void*> p(2 * (size_t)m);
-      for (uint32_t c = 0; c < m; c++) {
-        p[c] = h_eval[c0 + c];
-        p[m + c] = h_coeffs[c0 + c];
-      }
-      VX_HIP(hipMemcpyAsync(d.p, p.data(), p.size() * sizeof(void*), hipMemcpyHostToDevice, S(st)));
-      uint32_t* const* dst = static_cast<uint32_t* const*>(d.p);
-      ntt_forward_cols(dst, m, r, S(st), reinterpret_cast<const uint32_t* const*>(dst + m), log2u(coeff_n));
-      VX_HIP(hipStreamSynchronize(S(st)));
-    }
+    ntt_cols(h_eval, h_coeffs, n_cols, S(st),
+             [&](const NttCols& c) { ntt_forward_cols(c, r, S(st), log2u(coeff_n)); });
   });
 }
 
@@ -1394,8 +1400,8 @@ int vx_bit_reverse_m31_batch(const uint32_t* const* h_src, uint32_t* const* h_ds
   });
 }
 
-static LeafSrc lifted_src(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
-                          uint32_t lifting_log, DeviceBuf& table) {
+static std::vector<LiftCol> lifted_cols(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
+                                        uint32_t lifting_log) {
   require(h_cols && h_log_sizes && n_cols >= 1 && lifting_log >= 1 && lifting_log <= 31, "lifted: bad arguments");
   std::vector<LiftCol> lc(n_cols);
   for (uint32_t c = 0; c < n_cols; c++) {
@@ -1403,12 +1409,16 @@ static LeafSrc lifted_src(const uint32_t* const* h_cols, const uint32_t* h_log_s
     require(c == 0 || h_log_sizes[c] >= h_log_sizes[c - 1], "lifted: columns must be sorted by ascending size");
     lc[c] = {h_cols[c], h_log_sizes[c], 0};
   }
-  table = DeviceBuf(sizeof(LiftCol) * n_cols);
-  VX_HIP(hipMemcpy(table.p, lc.data(), sizeof(LiftCol) * n_cols, hipMemcpyHostToDevice));
+  return lc;
+}
+
+static LeafSrc lifted_src(const std::vector<LiftCol>& lc, uint32_t lifting_log, DeviceBuf& table) {
+  table = DeviceBuf(sizeof(LiftCol) * lc.size());
+  VX_HIP(hipMemcpy(table.p, lc.data(), sizeof(LiftCol) * lc.size(), hipMemcpyHostToDevice));
   LeafSrc L{};
   L.kind = LEAF_LIFTED;
   L.lift = static_cast<const LiftCol*>(table.p);
-  L.lift_n = n_cols;
+  L.lift_n = (uint32_t)lc.size();
   L.lift_log = lifting_log;
   return L;
 }
@@ -1417,9 +1427,12 @@ int vx_build_leaves_lifted(const uint32_t* const* h_cols, const uint32_t* h_log_
                            uint32_t lifting_log_size, uint32_t* d_hashes, vx_stream_t st) {
   return guard([&] {
     require(d_hashes != nullptr, "lifted: null output");
+    const std::vector<LiftCol> lc = lifted_cols(h_cols, h_log_sizes, n_cols, lifting_log_size);
     DeviceBuf table;
-    LeafSrc L = lifted_src(h_cols, h_log_sizes, n_cols, lifting_log_size, table);
-    merkle_lifted_leaves(L, d_hashes, S(st));
+    if (n_cols <= LIFT_ARG_COLS)
+      merkle_lifted_leaves(lc.data(), n_cols, lifting_log_size, d_hashes, S(st));
+    else
+      merkle_lifted_leaves(lifted_src(lc, lifting_log_size, table), d_hashes, S(st));
     VX_HIP(hipStreamSynchronize(S(st)));
   });
 }
@@ -1431,7 +1444,7 @@ int vx_merkle_root_lifted(const uint32_t* const* h_cols, const uint32_t* h_log_s
     const uint32_t lg = h_log_sizes[n_cols - 1];
     require(lg >= 4, "lifted: the largest column needs >= 16 rows");
     DeviceBuf table;
-    LeafSrc L = lifted_src(h_cols, h_log_sizes, n_cols, lg, table);
+    LeafSrc L = lifted_src(lifted_cols(h_cols, h_log_sizes, n_cols, lg), lg, table);
     // only the levels from the tile size up are stored (the tile roots and above)
     const uint32_t tile = merkle_tile_log(L, lg);
     TreeLevels T{};

@@ -254,17 +254,24 @@ __device__ __forceinline__ uint32_t ldg_at(const uint32_t* base, uint32_t byte_o
 // the update cost 4 VALU instructions per column, about 9 % of the lifted
 // tree's instructions; the empty asm statement keeps the compiler from
 // turning the branch into selects.)
+// The columns are a device array, or an array in the kernel's own arguments.
+struct LiftArgs {
+  LiftCol col[LIFT_ARG_COLS];
+};
+__device__ __forceinline__ LiftCol lift_col(const LiftCol* cols, uint32_t c) { return ld_uniform(cols + c); }
+__device__ __forceinline__ LiftCol lift_col(const LiftArgs& cols, uint32_t c) { return cols.col[c]; }
 struct LiftCursor {
   uint32_t log, off;
 };
-__device__ __forceinline__ void lifted_block(const LiftCol* cols, uint32_t n, uint32_t S, uint32_t i, uint32_t base,
+template <typename Cols>
+__device__ __forceinline__ void lifted_block(const Cols& cols, uint32_t n, uint32_t S, uint32_t i, uint32_t base,
                                              LiftCursor& cur, uint32_t (&m)[16]) {
 #pragma unroll
   for (uint32_t j = 0; j < 16; j++) {
     const uint32_t c = base + j;
     m[j] = 0;
     if (c < n) {
-      const LiftCol col = ld_uniform(cols + c);
+      const LiftCol col = lift_col(cols, c);
       if (col.log_n != cur.log) {
         asm volatile("" ::: "memory");
         cur.log = col.log_n;
@@ -274,8 +281,8 @@ __device__ __forceinline__ void lifted_block(const LiftCol* cols, uint32_t n, ui
     }
   }
 }
-template <bool WIDE>
-__device__ __forceinline__ void lifted_leaf_cols(const LiftCol* cols, uint32_t n, uint32_t S, uint64_t idx,
+template <bool WIDE, typename Cols>
+__device__ __forceinline__ void lifted_leaf_cols(const Cols& cols, uint32_t n, uint32_t S, uint64_t idx,
                                                  uint32_t (&h)[8]) {
   auto compress = [&](const uint32_t (&m)[16], uint32_t t, bool last) {
     if constexpr (WIDE) b2_compress_wide(h, m, t, last);
@@ -303,7 +310,7 @@ __device__ __forceinline__ void lifted_leaf_cols(const LiftCol* cols, uint32_t n
       const uint32_t c = base + j;
       uint32_t v = 0;
       if (c < n) {
-        const LiftCol col = ld_uniform(cols + c);
+        const LiftCol col = lift_col(cols, c);
         v = as_global(col.p)[lifted_row(idx, S, col.log_n)];
       }
       m[j] = v;
@@ -1289,20 +1296,35 @@ void merkle_leaf_pairs(const LeafSrc& L, uint64_t n_leaves, uint32_t* parents, h
   VX_HIP(hipGetLastError());
 }
 
-template <bool WIDE>
-__global__ void k_lifted_leaves(LeafSrc L, uint64_t n, uint32_t* hashes) {
+// Cols: the column table's device address, or the table itself in the
+// arguments. The latter spares a call its allocation, pageable upload and free.
+template <bool WIDE, typename Cols>
+__global__ void k_lifted_leaves(Cols cols, uint32_t n_cols, uint32_t lift_log, uint32_t* hashes) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= 1ull << lift_log) return;
   uint32_t h[8];
-  lifted_leaf<WIDE>(L, i, h);
+  lifted_leaf_cols<WIDE>(cols, n_cols, lift_log, i, h);
   store_node(hashes + 8 * i, h);
 }
-void merkle_lifted_leaves(const LeafSrc& L, uint32_t* hashes, hipStream_t s) {
-  check_leaf(L, L.lift_log);
-  const uint64_t n = 1ull << L.lift_log;
-  hipLaunchKernelGGL(wide_grid(n / 256) ? k_lifted_leaves<true> : k_lifted_leaves<false>, dim3((uint32_t)((n + 255) / 256)),
-                     dim3(256), 0, s, L, n, hashes);
+
+template <typename Cols>
+static void launch_lifted_leaves(const Cols& cols, uint32_t n_cols, uint32_t lift_log, uint32_t* hashes,
+                                 hipStream_t s) {
+  const uint64_t n = 1ull << lift_log;
+  hipLaunchKernelGGL(wide_grid(n / 256) ? (k_lifted_leaves<true, Cols>) : (k_lifted_leaves<false, Cols>),
+                     dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, cols, n_cols, lift_log, hashes);
   VX_HIP(hipGetLastError());
+}
+
+void merkle_lifted_leaves(const LeafSrc& L, uint32_t* hashes, hipStream_t s) {
+  launch_lifted_leaves(L.lift, L.lift_n, L.lift_log, hashes, s);
+}
+
+void merkle_lifted_leaves(const LiftCol* h_cols, uint32_t n_cols, uint32_t lift_log, uint32_t* hashes, hipStream_t s) {
+  require(n_cols >= 1 && n_cols <= LIFT_ARG_COLS, "lifted: too many columns for the kernel's arguments");
+  LiftArgs a{};
+  for (uint32_t c = 0; c < n_cols; c++) a.col[c] = h_cols[c];
+  launch_lifted_leaves(a, n_cols, lift_log, hashes, s);
 }
 
 // ------------------------------------------------------------- decommitment

@@ -14,6 +14,8 @@
 // takes two passes. The LDE's first log(N/n) evaluate layers only copy the
 // zero-padded coefficients, so the first pass reads coefficient i & (n-1)
 // directly and those layers are never executed.
+#include <type_traits>
+
 #include "vx_internal.h"
 #include "vx_issue.h"
 
@@ -28,8 +30,19 @@ static constexpr uint32_t NTT_STRIDED_MAX = 10; // bits per strided pass (>= 16 
 //             butterfly t uses +-L0[(t >> 1) ^ 1], negated when t & 3 is 1 or 2
 //             (that is (y, -y, -x, x)[t & 3] of the pair (L0[2p], L0[2p + 1]),
 //             p = t >> 2, cuda/circle_ntt_stwo.cu:214-234);
-//   NTT_COLS  column blockIdx.y of the batch is cols[blockIdx.y] (in place).
-enum : int { NTT_STWO = 1, NTT_COLS = 2 };
+//   NTT_COLS  column blockIdx.y of the batch has an address of its own, given
+//             in the kernel's arguments (at most NTT_ARG_COLS columns: nothing
+//             is allocated or uploaded) or in a device array.
+// (The enumeration has a name: it is part of the kernels' mangled names, which
+// the host and the device compilation must spell alike.)
+enum NttMode : int { NTT_STWO = 1, NTT_COLS = 2 };
+struct NoCols {};
+struct ColPtrs {
+  uint32_t* dst[NTT_ARG_COLS];
+  const uint32_t* src[NTT_ARG_COLS];  // the first pass's sources (null: in place)
+};
+template <int MODE>
+using ColArgs = std::conditional_t<(MODE & NTT_COLS) != 0, ColPtrs, NoCols>;
 
 struct PassArgs {
   const uint32_t* tw[16];  // twiddle table of bit j0 + b, for local bit b
@@ -37,8 +50,8 @@ struct PassArgs {
   uint64_t src_mask;
   uint32_t scale;          // output multiplier (1 = none)
   uint64_t dst_stride, src_stride;  // words between the columns of a batch (blockIdx.y)
-  uint32_t* const* cols;   // NTT_COLS: device array of column pointers (destinations)
-  const uint32_t* const* src_cols;  // NTT_COLS: source columns, or null to read the destinations
+  uint32_t* const* cols;   // NTT_COLS: device array of column pointers (destinations), null: in the arguments
+  const uint32_t* const* src_cols;  // NTT_COLS: with cols, source columns, or null to read the destinations
 };
 
 // stwo circle twiddle of circle butterfly h from line layer 0.
@@ -48,11 +61,13 @@ __device__ __forceinline__ uint32_t stwo_circle_tw(const uint32_t* l0, uint64_t 
 }
 
 template <bool FWD, int MODE>
-__global__ __launch_bounds__(NTT_THREADS) void k_ntt_pass(uint32_t* dst, const uint32_t* src, PassArgs a) {
+__global__ __launch_bounds__(NTT_THREADS) void k_ntt_pass(uint32_t* dst, const uint32_t* src, PassArgs a,
+                                                            ColArgs<MODE> cp) {
   extern __shared__ uint32_t lds[];
   if constexpr ((MODE & NTT_COLS) != 0) {
-    dst = ld_uniform(a.cols + blockIdx.y);
-    src = a.src_cols ? ld_uniform(a.src_cols + blockIdx.y) : dst;
+    dst = a.cols ? ld_uniform(a.cols + blockIdx.y) : cp.dst[blockIdx.y];
+    src = a.cols ? (a.src_cols ? ld_uniform(a.src_cols + blockIdx.y) : nullptr) : cp.src[blockIdx.y];
+    if (!src) src = dst;
   } else {
     dst += blockIdx.y * a.dst_stride;
     src += blockIdx.y * a.src_stride;
@@ -131,8 +146,8 @@ struct RadixArgs {
   uint64_t src_mask;
   uint32_t scale;
   uint64_t dst_stride, src_stride;
-  uint32_t* const* cols;   // NTT_COLS: device array of column pointers (destinations)
-  const uint32_t* const* src_cols;  // NTT_COLS: source columns, or null to read the destinations
+  uint32_t* const* cols;   // NTT_COLS: as in PassArgs
+  const uint32_t* const* src_cols;
   uint32_t launch_order;   // 1: tile b runs as workgroup b (else XCD-contiguous ranges)
 };
 
@@ -567,11 +582,13 @@ static int radix_shape(const RadixArgs& r) {
 }
 
 template <bool FWD, int MODE, int SHAPE>
-__global__ __launch_bounds__(RX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_radix(uint32_t* dst, const uint32_t* src, RadixArgs a) {
+__global__ __launch_bounds__(RX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_radix(uint32_t* dst, const uint32_t* src, RadixArgs a,
+                                                              ColArgs<MODE> cp) {
   __shared__ uint32_t lds[1u << RX_E_BITS];
   if constexpr ((MODE & NTT_COLS) != 0) {
-    dst = ld_uniform(a.cols + blockIdx.y);
-    src = a.src_cols ? ld_uniform(a.src_cols + blockIdx.y) : dst;
+    dst = a.cols ? ld_uniform(a.cols + blockIdx.y) : cp.dst[blockIdx.y];
+    src = a.cols ? (a.src_cols ? ld_uniform(a.src_cols + blockIdx.y) : nullptr) : cp.src[blockIdx.y];
+    if (!src) src = dst;
   } else {
     dst += blockIdx.y * a.dst_stride;
     src += blockIdx.y * a.src_stride;
@@ -626,25 +643,30 @@ static const uint32_t* bit_table(const TwiddleRef& tw, uint32_t j) {
 struct Batch {
   uint32_t n_cols;
   uint64_t dst_stride, src_stride;
-  uint32_t* const* cols;  // device column pointers, or null for strided columns
+  uint32_t* const* cols;  // device column pointers, or null
   const uint32_t* const* src_cols;  // with cols: the first pass's source columns (null: in place)
+  const ColPtrs* args;    // column pointers for the kernel's arguments, or null (neither: strided columns)
 };
 
-using RadixKernel = void (*)(uint32_t*, const uint32_t*, RadixArgs);
-using PassKernel = void (*)(uint32_t*, const uint32_t*, PassArgs);
-#define VX_RX_MODES(F, S) {k_ntt_radix<F, 0, S>, k_ntt_radix<F, 1, S>, k_ntt_radix<F, 2, S>, k_ntt_radix<F, 3, S>}
-static RadixKernel radix_kernel(bool fwd, int mode, int shape) {
-  static const RadixKernel k[2][3][4] = {
-      {VX_RX_MODES(false, RX_GENERIC), VX_RX_MODES(false, RX_CONTIG), VX_RX_MODES(false, RX_STRIDED)},
-      {VX_RX_MODES(true, RX_GENERIC), VX_RX_MODES(true, RX_CONTIG), VX_RX_MODES(true, RX_STRIDED)}};
-  return k[fwd ? 1 : 0][shape][mode];
+template <int MODE>
+using RadixKernel = void (*)(uint32_t*, const uint32_t*, RadixArgs, ColArgs<MODE>);
+template <int MODE>
+using PassKernel = void (*)(uint32_t*, const uint32_t*, PassArgs, ColArgs<MODE>);
+// MODE0: NTT_COLS or 0; the stwo flag is a run-time choice
+template <int MODE0>
+static RadixKernel<MODE0> radix_kernel(bool fwd, bool stwo, int shape) {
+#define VX_RX(F, S) {k_ntt_radix<F, MODE0, S>, k_ntt_radix<F, MODE0 | NTT_STWO, S>}
+  static const RadixKernel<MODE0> k[2][3][2] = {
+      {VX_RX(false, RX_GENERIC), VX_RX(false, RX_CONTIG), VX_RX(false, RX_STRIDED)},
+      {VX_RX(true, RX_GENERIC), VX_RX(true, RX_CONTIG), VX_RX(true, RX_STRIDED)}};
+#undef VX_RX
+  return k[fwd ? 1 : 0][shape][stwo ? 1 : 0];
 }
-#undef VX_RX_MODES
-static PassKernel pass_kernel(bool fwd, int mode) {
-  static const PassKernel k[2][4] = {
-      {k_ntt_pass<false, 0>, k_ntt_pass<false, 1>, k_ntt_pass<false, 2>, k_ntt_pass<false, 3>},
-      {k_ntt_pass<true, 0>, k_ntt_pass<true, 1>, k_ntt_pass<true, 2>, k_ntt_pass<true, 3>}};
-  return k[fwd ? 1 : 0][mode];
+template <int MODE0>
+static PassKernel<MODE0> pass_kernel(bool fwd, bool stwo) {
+  static const PassKernel<MODE0> k[2][2] = {{k_ntt_pass<false, MODE0>, k_ntt_pass<false, MODE0 | NTT_STWO>},
+                                            {k_ntt_pass<true, MODE0>, k_ntt_pass<true, MODE0 | NTT_STWO>}};
+  return k[fwd ? 1 : 0][stwo ? 1 : 0];
 }
 
 // Arguments of a 16384-element radix pass over bits [j0, j0 + k) with
@@ -693,7 +715,10 @@ static void launch_pass(bool fwd, uint32_t* dst, const uint32_t* src, uint64_t s
   a.cols = bt.cols;
   a.src_cols = bt.src_cols;
   require(bt.n_cols >= 1 && bt.n_cols <= 65535, "ntt: 1..65535 columns per batch");
-  const int mode = (tw.stwo_circle ? NTT_STWO : 0) | (bt.cols ? NTT_COLS : 0);
+  const bool stwo = tw.stwo_circle != 0, cols = bt.cols || bt.args;
+  require(!bt.args || bt.n_cols <= NTT_ARG_COLS, "ntt: too many columns for the kernel's arguments");
+  static const ColPtrs none{};
+  const ColPtrs& cp = bt.args ? *bt.args : none;
   const uint32_t e_log = k + cbits;
   const uint64_t grid = 1ull << (log_n - e_log);
   if (e_log == RX_E_BITS) {
@@ -703,14 +728,19 @@ static void launch_pass(bool fwd, uint32_t* dst, const uint32_t* src, uint64_t s
     r.cols = bt.cols;
     r.src_cols = bt.src_cols;
     r.launch_order = launch_order;
-    hipLaunchKernelGGL(radix_kernel(fwd, mode, radix_shape(r)), dim3((uint32_t)grid, bt.n_cols), dim3(RX_THREADS), 0,
-                       s, dst, src, r);
+    const dim3 g((uint32_t)grid, bt.n_cols);
+    if (cols)
+      hipLaunchKernelGGL(radix_kernel<NTT_COLS>(fwd, stwo, radix_shape(r)), g, dim3(RX_THREADS), 0, s, dst, src, r, cp);
+    else
+      hipLaunchKernelGGL(radix_kernel<0>(fwd, stwo, radix_shape(r)), g, dim3(RX_THREADS), 0, s, dst, src, r, NoCols{});
     VX_HIP(hipGetLastError());
     return;
   }
   const uint32_t threads = e_log >= 10 ? NTT_THREADS : (e_log >= 7 ? (1u << (e_log - 1)) : 64u);
   const size_t lds = (size_t)4 << e_log;
-  hipLaunchKernelGGL(pass_kernel(fwd, mode), dim3((uint32_t)grid, bt.n_cols), dim3(threads), lds, s, dst, src, a);
+  const dim3 g((uint32_t)grid, bt.n_cols);
+  if (cols) hipLaunchKernelGGL(pass_kernel<NTT_COLS>(fwd, stwo), g, dim3(threads), lds, s, dst, src, a, cp);
+  else hipLaunchKernelGGL(pass_kernel<0>(fwd, stwo), g, dim3(threads), lds, s, dst, src, a, NoCols{});
   VX_HIP(hipGetLastError());
 }
 
@@ -727,6 +757,15 @@ static uint32_t strided_passes(uint32_t strided_bits, const NttPlan& plan) {
   return n;
 }
 
+static ColPtrs col_ptrs(uint32_t* const* h_cols, uint32_t n_cols, const uint32_t* const* h_src_cols) {
+  ColPtrs c{};
+  for (uint32_t k = 0; k < n_cols; k++) {
+    c.dst[k] = h_cols[k];
+    c.src[k] = h_src_cols ? h_src_cols[k] : nullptr;
+  }
+  return c;
+}
+
 static void forward_passes(uint32_t* data, const uint32_t* src, uint64_t src_mask, const TwiddleRef& tw,
                            uint32_t eff_bits, hipStream_t s, Batch bt, const NttPlan& plan) {
   const uint32_t log_n = tw.log_n;
@@ -737,6 +776,7 @@ static void forward_passes(uint32_t* data, const uint32_t* src, uint64_t src_mas
   const uint32_t n_strided = strided_passes(strided_bits, plan);
   const uint32_t* cur = src;
   uint64_t mask = src_mask;
+  ColPtrs in_place;
   for (uint32_t p = 0; p < n_strided; p++) {
     uint32_t k = (top - contig) / (n_strided - p);  // balanced chunks
     uint32_t j0 = top - k;
@@ -746,6 +786,10 @@ static void forward_passes(uint32_t* data, const uint32_t* src, uint64_t src_mas
     mask = (1ull << log_n) - 1;
     bt.src_stride = dst_stride;
     bt.src_cols = nullptr;  // later passes work in place on the destinations
+    if (bt.args && p == 0) {
+      in_place = col_ptrs(bt.args->dst, bt.n_cols, nullptr);
+      bt.args = &in_place;
+    }
   }
   launch_pass(true, data, cur, mask, tw, 0, contig, 0, 1u, bt, s, plan.order);
 }
@@ -760,7 +804,7 @@ void ntt_forward(uint32_t* data, const uint32_t* src, uint64_t src_mask, const T
           "ntt_forward: source length must be a power of two covering the transformed bits");
   require(n_cols == 1 || (dst_stride >= (1ull << log_n) && src_stride >= src_mask + 1),
           "ntt_forward: batch columns must not overlap");
-  const Batch bt{n_cols, dst_stride, src_stride, nullptr, nullptr};
+  const Batch bt{n_cols, dst_stride, src_stride, nullptr, nullptr, nullptr};
   const NttKey key{true, tw.log_n, eff_bits, n_cols, tw.stwo_circle != 0};
   // out of place, the first pass reads src intact, so the candidates run on
   // the caller's buffers; in place they run on a scratch buffer of the same
@@ -786,13 +830,18 @@ void ntt_forward(uint32_t* data, const uint32_t* src, uint64_t src_mask, const T
   forward_passes(data, src, src_mask, tw, eff_bits, s, bt, plan);
 }
 
-void ntt_forward_cols(uint32_t* const* d_cols, uint32_t n_cols, const TwiddleRef& tw, hipStream_t s,
-                      const uint32_t* const* d_src_cols, uint32_t src_log_n) {
-  require(d_cols != nullptr && tw.log_n >= 1 && tw.log_n <= 31, "ntt_forward_cols: bad arguments");
-  const uint32_t eff = d_src_cols ? src_log_n : tw.log_n;
+void ntt_forward_cols(const NttCols& cols, const TwiddleRef& tw, hipStream_t s, uint32_t src_log_n) {
+  require(tw.log_n >= 1 && tw.log_n <= 31, "ntt_forward_cols: bad arguments");
+  const uint32_t eff = cols.src ? src_log_n : tw.log_n;
   require(eff >= 1 && eff <= tw.log_n, "ntt_forward_cols: source size must be 2..2^log_n");
-  const NttPlan plan = known_ntt_plan(NttKey{true, tw.log_n, eff, n_cols, tw.stwo_circle != 0});
-  forward_passes(nullptr, nullptr, (1ull << eff) - 1, tw, eff, s, Batch{n_cols, 0, 0, d_cols, d_src_cols}, plan);
+  const NttPlan plan = known_ntt_plan(NttKey{true, tw.log_n, eff, cols.n, tw.stwo_circle != 0});
+  const uint64_t mask = (1ull << eff) - 1;
+  if (cols.on_device) {
+    forward_passes(nullptr, nullptr, mask, tw, eff, s, Batch{cols.n, 0, 0, cols.dst, cols.src, nullptr}, plan);
+  } else {
+    const ColPtrs c = col_ptrs(cols.dst, cols.n, cols.src);
+    forward_passes(nullptr, nullptr, mask, tw, eff, s, Batch{cols.n, 0, 0, nullptr, nullptr, &c}, plan);
+  }
 }
 
 static void inverse_passes(uint32_t* data, const TwiddleRef& tw, hipStream_t s, const Batch& bt,
@@ -819,7 +868,7 @@ void ntt_inverse(uint32_t* data, const TwiddleRef& tw, hipStream_t s, uint32_t n
   require(aligned16(data) && stride % 4 == 0, "ntt: columns must be 16-byte aligned");
   require(log_n >= 1 && log_n <= 31, "ntt_inverse: bad size");
   require(n_cols == 1 || stride >= (1ull << log_n), "ntt_inverse: batch columns must not overlap");
-  const Batch bt{n_cols, stride, stride, nullptr, nullptr};
+  const Batch bt{n_cols, stride, stride, nullptr, nullptr, nullptr};
   const NttKey key{false, log_n, log_n, n_cols, tw.stwo_circle != 0};
   // in place: the candidates are timed on a scratch buffer of the same
   // shape (allocated only when this shape is measured)
@@ -839,10 +888,15 @@ void ntt_inverse(uint32_t* data, const TwiddleRef& tw, hipStream_t s, uint32_t n
   inverse_passes(data, tw, s, bt, plan);
 }
 
-void ntt_inverse_cols(uint32_t* const* d_cols, uint32_t n_cols, const TwiddleRef& tw, hipStream_t s) {
-  require(d_cols != nullptr && tw.log_n >= 1 && tw.log_n <= 31, "ntt_inverse_cols: bad arguments");
-  inverse_passes(nullptr, tw, s, Batch{n_cols, 0, 0, d_cols, nullptr},
-                 known_ntt_plan(NttKey{false, tw.log_n, tw.log_n, n_cols, tw.stwo_circle != 0}));
+void ntt_inverse_cols(const NttCols& cols, const TwiddleRef& tw, hipStream_t s) {
+  require(tw.log_n >= 1 && tw.log_n <= 31, "ntt_inverse_cols: bad arguments");
+  const NttPlan plan = known_ntt_plan(NttKey{false, tw.log_n, tw.log_n, cols.n, tw.stwo_circle != 0});
+  if (cols.on_device) {
+    inverse_passes(nullptr, tw, s, Batch{cols.n, 0, 0, cols.dst, nullptr, nullptr}, plan);
+  } else {
+    const ColPtrs c = col_ptrs(cols.dst, cols.n, nullptr);
+    inverse_passes(nullptr, tw, s, Batch{cols.n, 0, 0, nullptr, nullptr, &c}, plan);
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -112,14 +112,22 @@ void ntt_forward(uint32_t* data, const uint32_t* src, uint64_t src_mask, const T
                  uint32_t eff_bits, hipStream_t s, uint32_t n_cols = 1, uint64_t dst_stride = 0,
                  uint64_t src_stride = 0);
 void ntt_inverse(uint32_t* data, const TwiddleRef& tw, hipStream_t s, uint32_t n_cols = 1, uint64_t stride = 0);
-// In-place transforms of n_cols columns of 2^log_n words each at arbitrary
-// (16-byte aligned) addresses: d_cols is a device array of column pointers.
-// Same passes as ntt_forward / ntt_inverse, one launch per pass for all columns.
-// With d_src_cols, the forward transform reads 2^src_log_n coefficients per
-// column from there, zero-padded (the LDE: the replication layers are skipped).
-void ntt_forward_cols(uint32_t* const* d_cols, uint32_t n_cols, const TwiddleRef& tw, hipStream_t s,
-                      const uint32_t* const* d_src_cols = nullptr, uint32_t src_log_n = 0);
-void ntt_inverse_cols(uint32_t* const* d_cols, uint32_t n_cols, const TwiddleRef& tw, hipStream_t s);
+// In-place transforms of n columns of 2^log_n words each at arbitrary (16-byte
+// aligned) addresses; same passes as ntt_forward / ntt_inverse, one launch per
+// pass for all columns. With src, the forward transform reads 2^src_log_n
+// coefficients per column from there, zero-padded (the LDE: the replication
+// layers are skipped). The pointer arrays are the host's, of at most
+// NTT_ARG_COLS columns, and travel in the kernels' arguments; or on_device, of
+// any number up to 65,535.
+constexpr uint32_t NTT_ARG_COLS = 128;
+struct NttCols {
+  uint32_t* const* dst;
+  const uint32_t* const* src;  // null: in place
+  uint32_t n;
+  bool on_device;
+};
+void ntt_forward_cols(const NttCols& cols, const TwiddleRef& tw, hipStream_t s, uint32_t src_log_n = 0);
+void ntt_inverse_cols(const NttCols& cols, const TwiddleRef& tw, hipStream_t s);
 // Uneven batched LDE (columns of log sizes 14..24): host-built work lists
 // (lde_batch_build) uploaded by the caller, then four launches.
 struct LdeBatchCol {
@@ -353,7 +361,11 @@ void merkle_reduce_to_root(const uint32_t* nodes, uint32_t* root, uint32_t n_nod
 void merkle_root_small(const LeafSrc& leaf, uint32_t log_n, uint32_t* root_out, hipStream_t s);
 void merkle_leaf_pairs(const LeafSrc& leaf, uint64_t n_leaves, uint32_t* parents, hipStream_t s);
 // Every leaf hash of a lifted tree (cuda_build_leaves_lifted semantics).
+// Lifted leaf hashes; the columns in device memory, or on the host (at most
+// LIFT_ARG_COLS: they travel in the kernel's arguments).
 void merkle_lifted_leaves(const LeafSrc& leaf, uint32_t* hashes, hipStream_t s);
+constexpr uint32_t LIFT_ARG_COLS = 128;
+void merkle_lifted_leaves(const LiftCol* h_cols, uint32_t n_cols, uint32_t lift_log, uint32_t* hashes, hipStream_t s);
 // Cairo VM AIR quotient (cairo.hip).
 void cairo_quotient(const CairoArgs& a, uint64_t rows, hipStream_t s);
 void cairo_vanishing(uint32_t ix, uint32_t iy, uint32_t sx, uint32_t sy, uint32_t* out, uint32_t log_eval,
