@@ -45,3 +45,21 @@ def test_chunks_match_oracle(logs, fill):
             # a smaller column takes the last L factors
             seen[key] = po.eval_at_point_factors(c, factors[4 * (max_log - L):])
         assert tuple(int(v) for v in got[k]) == seen[key], (k, L)
+
+
+@pytest.mark.parametrize("n_cols", [1, 2, 3, 127, 128, 129, 255])
+def test_mixed_values(n_cols):
+    """The transcript's message at the edges of its blocks (16 words) and of
+    the 64 blocks laid out at a time (127 columns are 64 blocks)."""
+    print("oods mix", n_cols, flush=True)
+    rng = np.random.default_rng(n_cols)
+    cols = [rng.integers(0, P, 8, dtype=np.uint32) for _ in range(n_cols)]
+    ch = po.PyChannel()
+    ch.mix_digest([n_cols, 2, 7, 1, 8, 2, 8, 1])
+    words = lambda: np.concatenate([np.frombuffer(ch.state, np.uint32), [ch.c.n_draws]]).astype(np.uint32)
+    bufs, d_ch, pts, vals = [dev(c) for c in cols], dev(words()), empty(16), empty(8 * n_cols)
+    call("vx_oods_sample", ptr(d_ch), (C.c_void_p * n_cols)(*[b.ptr for b in bufs]), (C.c_uint32 * n_cols)(*[3] * n_cols),
+         n_cols, 5, ptr(pts), ptr(vals), None)
+    want_pts, want_vals = ch.oods_sample(cols, 5)
+    assert np.array_equal(host(pts), want_pts) and np.array_equal(host(vals), want_vals)
+    assert np.array_equal(host(d_ch), words())

@@ -431,13 +431,19 @@ __global__ __launch_bounds__(64) void k_eval_sum(EvalCols a, uint32_t n_wgs, con
   }
 }
 
-// np points (1 or 2): factors holds np tables of 4 max_log_n words back to
-// back (4 words when max_log_n is 0), results np arrays of n_cols QM31.
-// The work is enqueued on s; `ws` is the caller's to free when it is done.
-static void eval_batch_points(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
-                              const uint32_t* factors, uint32_t np, uint32_t max_log_n, uint32_t* results,
-                              DeviceBuf& ws, hipStream_t s) {
-  if (n_cols == 0) return;
+// The split of a batch into workgroups and its workspace, after checking it.
+struct EvalPlan {
+  EvalTables T;
+  uint32_t cpw_log;
+  uint64_t wgs;
+  uint64_t ws_words() const { return T.words() + 4ull * T.np * wgs; }
+};
+static uint32_t eval_wgs_of(uint32_t L, uint32_t cpw_log) {
+  const uint32_t c = L > EV_BIG_LOG ? L - EV_BIG_LOG : 0;
+  return c > cpw_log ? 1u << (c - cpw_log) : 1u;
+}
+static EvalPlan eval_plan(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols, uint32_t np,
+                          uint32_t max_log_n) {
   require(np == 1 || np == 2, "eval_at_point_batch: one or two points");
   require(max_log_n <= 31, "eval_at_point_batch: max_log_n must be <= 31");
   uint64_t total = 0;
@@ -455,15 +461,21 @@ static void eval_batch_points(const uint32_t* const* h_cols, const uint32_t* h_l
   // once per workgroup, so no more workgroups than keep the chip full.
   uint32_t cpw_log = 0;
   while ((total >> cpw_log) > EV_MAX_WGS) cpw_log++;
-  auto wgs_of = [&](uint32_t L) {
-    const uint32_t c = L > EV_BIG_LOG ? L - EV_BIG_LOG : 0;
-    return c > cpw_log ? 1u << (c - cpw_log) : 1u;
-  };
   uint64_t wgs = 0;
-  for (uint32_t k = 0; k < n_cols; k++) wgs += wgs_of(h_log_sizes[k]);
-  const EvalTables T{np, top > EV_BIG_LOG ? top - EV_BIG_LOG : 0};
-  ws = DeviceBuf(4 * T.words() + 16ull * np * wgs);
-  uint32_t* tables = ws.u32();
+  for (uint32_t k = 0; k < n_cols; k++) wgs += eval_wgs_of(h_log_sizes[k], cpw_log);
+  return {EvalTables{np, top > EV_BIG_LOG ? top - EV_BIG_LOG : 0}, cpw_log, wgs};
+}
+
+// np points (1 or 2): factors holds np tables of 4 max_log_n words back to
+// back (4 words when max_log_n is 0), results np arrays of n_cols QM31.
+// The work is enqueued on s; the workspace (ws_words) must outlive it.
+static void eval_batch_points(const EvalPlan& plan, const uint32_t* const* h_cols, const uint32_t* h_log_sizes,
+                              uint32_t n_cols, const uint32_t* factors, uint32_t max_log_n, uint32_t* results,
+                              uint32_t* ws, hipStream_t s) {
+  const EvalTables& T = plan.T;
+  const uint32_t np = T.np, cpw_log = plan.cpw_log;
+  const uint64_t wgs = plan.wgs;
+  uint32_t* tables = ws;
   uint32_t* part = tables + T.words();
   const uint64_t entries = EV_TERMS + 1 + EV_WG + (1ull << T.g_log);
   hipLaunchKernelGGL(k_eval_tables, dim3((uint32_t)((entries + EV_WG - 1) / EV_WG), np), dim3(EV_WG), 0, s, factors,
@@ -480,7 +492,7 @@ static void eval_batch_points(const uint32_t* const* h_cols, const uint32_t* h_l
       a.col[k] = h_cols[k0 + k];
       a.log_n[k] = (uint8_t)h_log_sizes[k0 + k];
       a.first[k] = w;
-      w += wgs_of(h_log_sizes[k0 + k]);
+      w += eval_wgs_of(h_log_sizes[k0 + k], cpw_log);
     }
     if (np == 2)
       hipLaunchKernelGGL(k_eval_chunks<2>, dim3(w), dim3(EV_WG), 0, s, a, T, tables, part, (uint32_t)wgs);
@@ -495,8 +507,10 @@ static void eval_batch_points(const uint32_t* const* h_cols, const uint32_t* h_l
 
 void eval_at_point_batch(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
                          const uint32_t* factors, uint32_t max_log_n, uint32_t* results, hipStream_t s) {
-  DeviceBuf ws;
-  eval_batch_points(h_cols, h_log_sizes, n_cols, factors, 1, max_log_n, results, ws, s);
+  if (n_cols == 0) return;
+  const EvalPlan plan = eval_plan(h_cols, h_log_sizes, n_cols, 1, max_log_n);
+  DeviceBuf ws(4 * plan.ws_words());
+  eval_batch_points(plan, h_cols, h_log_sizes, n_cols, factors, max_log_n, results, ws.u32(), s);
   VX_HIP(hipStreamSynchronize(s));  // the workspace is freed on return
 }
 
@@ -600,35 +614,73 @@ __global__ void k_oods_point(uint32_t* ch_words, uint32_t trace_log, uint32_t ma
 
 // Channel::mix_felts (src/channel.rs:46-59) of the sampled values: the
 // message is state || values; it is a dependent chain of compressions, which
-// the four lanes of a quad share (b2_compress_x4, about 430 instructions per
-// lane and block instead of 960). A block's words are loaded while the block
-// before it is compressed. One wavefront; lanes 0..3 write the new state.
-__global__ __launch_bounds__(64) void k_oods_mix(uint32_t* ch_words, const uint32_t* values, uint32_t n_felts) {
+// the four lanes of a quad share. All words are known beforehand, so the
+// workgroup lays MIX_BLOCKS blocks at a time out in LDS in schedule order, one
+// 16-byte read per round and lane, and one wavefront runs the chain over them
+// with the next block's ten reads in flight: 300 instructions per lane and
+// block instead of 430 with the words selected from registers. Bound by that
+// chain: 64 columns (33 blocks) 36 -> 23 us, of which the layout is about 3.
+static constexpr uint32_t MIX_BLOCKS = 64, MIX_THREADS = 640;
+struct MixWords {
+  uint8_t at[160];  // message word of schedule entry 16 round + 4 lane + k
+};
+constexpr MixWords make_mix_words() {
+  MixWords t{};
+  for (uint32_t e = 0; e < 160; e++) t.at[e] = (uint8_t)quad_word(e / 4 % 4, 4 * (e / 16) + e % 4);
+  return t;
+}
+__constant__ const MixWords MIX_WORDS = make_mix_words();
+
+__global__ __launch_bounds__(MIX_THREADS) void k_oods_mix(uint32_t* ch_words, const uint32_t* values,
+                                                          uint32_t n_felts) {
+  __shared__ uint32_t msg[16 * MIX_BLOCKS];
+  __shared__ __align__(16) uint32_t sched[160 * MIX_BLOCKS];
   if (blockIdx.x != 0 || n_felts == 0) return;
-  const uint32_t q = threadIdx.x & 3u;
+  const uint32_t tid = threadIdx.x, q = tid & 3u, word = MIX_WORDS.at[tid % 160u];
   const bool q0 = q & 1, q1 = q & 2;
   uint32_t h_lo = sel4(q0, q1, VX_B2_IV0 ^ 0x01010020u, VX_B2_IV1, VX_B2_IV2, VX_B2_IV3);
   uint32_t h_hi = sel4(q0, q1, VX_B2_IV4, VX_B2_IV5, VX_B2_IV6, VX_B2_IV7);
-  const uint32_t nwords = 8 + 4 * n_felts;
-  uint32_t m[16], next[16];
-#pragma unroll
-  for (uint32_t k = 0; k < 16; k++) m[k] = k < 8 ? ch_words[k] : k < nwords ? values[k - 8] : 0u;
-  for (uint32_t at = 0;; at += 16) {
-    const bool last = nwords - at <= 16;
-    if (!last) {
-#pragma unroll
-      for (uint32_t k = 0; k < 16; k++) next[k] = at + 16 + k < nwords ? values[at + 8 + k] : 0u;
+  const uint64_t nwords = 8 + 4ull * n_felts;
+  const uint32_t n_blocks = (uint32_t)((nwords + 15) / 16);
+  for (uint32_t b0 = 0; b0 < n_blocks; b0 += MIX_BLOCKS) {
+    const uint32_t nb = n_blocks - b0 < MIX_BLOCKS ? n_blocks - b0 : MIX_BLOCKS;
+    __syncthreads();  // the chain is through with the blocks before
+    for (uint32_t k = tid; k < 16 * nb; k += MIX_THREADS) {
+      const uint64_t at = 16ull * b0 + k;
+      msg[k] = at < 8 ? ch_words[at] : at < nwords ? values[at - 8] : 0u;
     }
-    b2_compress_x4(h_lo, h_hi, m, last ? 4 * nwords : 4 * (at + 16), last, q);
-    if (last) break;
+    __syncthreads();
+    for (uint32_t b = tid / 160u; b < nb; b += MIX_THREADS / 160u) sched[160 * b + tid % 160u] = msg[16 * b + word];
+    __syncthreads();
+    if (tid < 64) {
+      const uint4* sq = reinterpret_cast<const uint4*>(sched) + q;
+      auto read = [&](uint4 (&w)[10], uint32_t b) {
+        // past the last block: the last one once more, unused
+        const uint4* sn = sq + 40 * (b < nb ? b : nb - 1);
 #pragma unroll
-    for (uint32_t k = 0; k < 16; k++) m[k] = next[k];
+        for (int r = 0; r < 10; r++) w[r] = sn[4 * r];
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto compress = [&](const uint4 (&w)[10], uint32_t b) {
+        const bool last = b0 + b + 1 == n_blocks;
+        b2_compress_x4(h_lo, h_hi, w, last ? (uint32_t)(4 * nwords) : 64 * (b0 + b + 1), last, q);
+      };
+      uint4 w0[10], w1[10];  // taken in turn: no copies
+      read(w0, 0);
+      for (uint32_t b = 0; b < nb; b += 2) {
+        read(w1, b + 1);
+        compress(w0, b);
+        if (b + 1 == nb) break;
+        read(w0, b + 2);
+        compress(w1, b + 1);
+      }
+    }
   }
-  if (threadIdx.x < 4) {
+  if (tid < 4) {
     ch_words[q] = h_lo;
     ch_words[4 + q] = h_hi;
   }
-  if (threadIdx.x == 0) ch_words[8] = 0;
+  if (tid == 0) ch_words[8] = 0;
 }
 
 void oods_sample(uint32_t* d_channel, const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
@@ -636,17 +688,21 @@ void oods_sample(uint32_t* d_channel, const uint32_t* const* h_cols, const uint3
   uint32_t max_log = 0;
   for (uint32_t k = 0; k < n_cols; k++) max_log = h_log_sizes[k] > max_log ? h_log_sizes[k] : max_log;
   const uint32_t fw = 4 * (max_log ? max_log : 1);
-  DeviceBuf fac(8ull * fw), ws;
-  uint32_t* fz = fac.u32();
+  // one allocation: both points' factors, then the evaluation's workspace
+  EvalPlan plan{};
+  if (n_cols) plan = eval_plan(h_cols, h_log_sizes, n_cols, 2, max_log);
+  const uint64_t ws_at = (2ull * fw + 63) & ~63ull;
+  DeviceBuf buf(4 * (ws_at + (n_cols ? plan.ws_words() : 0)));
+  uint32_t* fz = buf.u32();
   hipLaunchKernelGGL(k_oods_point, dim3(1), dim3(64), 0, s, d_channel, trace_log, max_log, d_points, fz, fz + fw);
   VX_HIP(hipGetLastError());
   if (n_cols) {
     // both points from one read of every column: values at z, then at z_next
-    eval_batch_points(h_cols, h_log_sizes, n_cols, fz, 2, max_log, d_values, ws, s);
-    hipLaunchKernelGGL(k_oods_mix, dim3(1), dim3(64), 0, s, d_channel, d_values, 2 * n_cols);
+    eval_batch_points(plan, h_cols, h_log_sizes, n_cols, fz, max_log, d_values, buf.u32() + ws_at, s);
+    hipLaunchKernelGGL(k_oods_mix, dim3(1), dim3(MIX_THREADS), 0, s, d_channel, d_values, 2 * n_cols);
     VX_HIP(hipGetLastError());
   }
-  VX_HIP(hipStreamSynchronize(s));  // the workspaces are freed on return
+  VX_HIP(hipStreamSynchronize(s));  // the workspace is freed on return
 }
 
 }  // namespace vx

@@ -151,6 +151,15 @@ struct QuadLds {
   }
 };
 
+// The ten rounds on a message a lane holds in its own schedule order.
+struct QuadSched {
+  const uint4 (&w)[10];
+  __device__ __forceinline__ void rounds(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) const {
+#pragma unroll
+    for (int r = 0; r < 10; r++) b2_round_x4(a, b, c, d, w[r].x, w[r].y, w[r].z, w[r].w);
+  }
+};
+
 // Single-block Blake2s of `t` message bytes (the final block; bytes past t
 // are zero in the message) by the four lanes of a quad, q = lane & 3. Returns
 // output words q and 4 + q in lo / hi.
@@ -177,18 +186,27 @@ __device__ __forceinline__ void b2_hash_x4_lds(const uint32_t* msg, const QuadOf
 // One compression of a chained hash by the four lanes of a quad: lane q
 // holds chaining words q and 4 + q in h_lo / h_hi and updates them; t is the
 // byte count up to and including this block, last marks the final block.
-// All four lanes pass the same 16 message words. Same function as
-// b2_compress.
-__device__ __forceinline__ void b2_compress_x4(uint32_t& h_lo, uint32_t& h_hi, const uint32_t (&m)[16], uint32_t t,
-                                               bool last, uint32_t q) {
+// All four lanes pass the same 16 message words, or each its own schedule of
+// them. Same function as b2_compress.
+template <typename W>
+__device__ __forceinline__ void b2_compress_x4_of(uint32_t& h_lo, uint32_t& h_hi, const W& words, uint32_t t, bool last,
+                                                  uint32_t q) {
   const bool q0 = q & 1, q1 = q & 2;
   uint32_t a = h_lo, b = h_hi;
   uint32_t c = sel4(q0, q1, VX_B2_IV0, VX_B2_IV1, VX_B2_IV2, VX_B2_IV3);
   uint32_t d = sel4(q0, q1, VX_B2_IV4, VX_B2_IV5, VX_B2_IV6, VX_B2_IV7) ^ (q == 0 ? t : 0u) ^
                (q == 2 && last ? 0xFFFFFFFFu : 0u);  // v12 ^= t, v14 ^= final
-  QuadRegs{m, q0, q1}.rounds(a, b, c, d);
+  words.rounds(a, b, c, d);
   h_lo ^= a ^ c;
   h_hi ^= b ^ d;
+}
+__device__ __forceinline__ void b2_compress_x4(uint32_t& h_lo, uint32_t& h_hi, const uint32_t (&m)[16], uint32_t t,
+                                               bool last, uint32_t q) {
+  b2_compress_x4_of(h_lo, h_hi, QuadRegs{m, (q & 1) != 0, (q & 2) != 0}, t, last, q);
+}
+__device__ __forceinline__ void b2_compress_x4(uint32_t& h_lo, uint32_t& h_hi, const uint4 (&w)[10], uint32_t t,
+                                               bool last, uint32_t q) {
+  b2_compress_x4_of(h_lo, h_hi, QuadSched{w}, t, last, q);
 }
 
 // LDS writes of a lane before, LDS reads of the wavefront's other lanes
