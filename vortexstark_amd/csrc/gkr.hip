@@ -94,48 +94,59 @@ __global__ __launch_bounds__(GKR_THREADS) void k_gkr_eq_pass(uint32_t* buf, cons
 
 // The whole eq table in one launch. Entry x of the reference's passes is
 // v prod_i (bit i of x ? y[k-1-i] : 1 - y[k-1-i]), a product that splits
-// over the index bits: each workgroup owns GKR_EQ_HPW consecutive values H
-// of the high bits (2^kl entries each), builds the low-bit factor table in
-// LDS by the same doubling passes (from 1), forms v times the high-bit
-// factors of its H values (one lane each), and writes their products, so
-// every entry costs one product and one 16-byte store. Field products are
-// exact, so the entries equal the pass-by-pass ones.
-constexpr uint32_t GKR_EQ_LO_MAX = 10;
-constexpr uint32_t GKR_EQ_HPW = 16;
+// over the index bits: the low kl <= 8 bits are a lane's own factor, the next
+// hb bits run over a workgroup's 2^hb values H, the rest is the workgroup's.
+// Every lane forms its low factor (kl products), every wavefront the
+// workgroup's factor (a tree product over lanes), 2^hb lanes the H values'
+// (hb products more), and an entry then costs one product and one 16-byte
+// store. Field products are exact, so the entries equal the pass-by-pass ones.
+// Serial products bind it up to about 2^20 entries: 2^20 took 24 us with
+// a table of 2^10 low factors built in LDS by ten passes with a barrier each
+// in 64 workgroups, 11.7 us so (3.3 for the stores alone).
+constexpr uint32_t GKR_EQ_LO_MAX = 8;  // 2^8 lanes
+constexpr uint32_t GKR_EQ_HB_MAX = 6;
+__device__ __forceinline__ qm31 eq_factor(const uint4* y, uint32_t k, uint32_t i, bool bit) {
+  const uint4 w = y[k - 1 - i];
+  const qm31 yi{{w.x, w.y, w.z, w.w}};
+  return bit ? yi : qm_one_minus(yi);
+}
 __global__ __launch_bounds__(GKR_THREADS) void k_gkr_eq_table(uint32_t* buf, const uint32_t* y, uint32_t k,
-                                                             uint32_t kl, uint32_t hpw, const uint32_t* v, bool a16) {
-  __shared__ uint4 lo[1u << GKR_EQ_LO_MAX];
-  __shared__ uint4 hi[GKR_EQ_HPW];
-  const uint32_t t = threadIdx.x;
-  const uint64_t H0 = (uint64_t)blockIdx.x * hpw;
-  if (t < hpw) {
-    const uint64_t H = H0 + t;
-    qm31 acc = ldq_arg(v);
-    for (uint32_t i = kl; i < k; i++) {
-      const qm31 yi = ldq_arg(y + 4 * (k - 1 - i));
-      acc = qm_mul_lazy(acc, ((H >> (i - kl)) & 1) ? yi : qm_one_minus(yi));
-    }
-    hi[t] = make_uint4(acc.v[0], acc.v[1], acc.v[2], acc.v[3]);
-  }
-  if (t == 0) lo[0] = make_uint4(1u, 0u, 0u, 0u);
+                                                             uint32_t kl, uint32_t hb, const uint32_t* v, bool a16) {
+  __shared__ uint4 ys[32];
+  __shared__ uint4 hi[1u << GKR_EQ_HB_MAX];
+  const uint32_t t = threadIdx.x, lane = t & 63u;
+  if (t < 4 * k) reinterpret_cast<uint32_t*>(ys)[t] = y[t];
+  const qm31 vq = ldq_arg(v);
   __syncthreads();
-  for (uint32_t i = 0; i < kl; i++) {
-    const uint32_t cur = 1u << i;
-    const qm31 yi = ldq_arg(y + 4 * (k - 1 - i));
-    for (uint32_t j = t; j < cur; j += GKR_THREADS) {
-      const uint4 e = lo[j];
-      const qm31 ev{{e.x, e.y, e.z, e.w}}, tt = qm_mul_lazy(ev, yi), d = qm_sub(ev, tt);
-      lo[cur + j] = make_uint4(tt.v[0], tt.v[1], tt.v[2], tt.v[3]);
-      lo[j] = make_uint4(d.v[0], d.v[1], d.v[2], d.v[3]);
-    }
-    __syncthreads();
+  const qm31 one{{1u, 0u, 0u, 0u}};
+  qm31 top = one;  // lane l: the factor of bit kl + hb + l
+  if (kl + hb + lane < k) top = eq_factor(ys, k, kl + hb + lane, (blockIdx.x >> lane) & 1u);
+#pragma unroll
+  for (int off = 16; off >= 1; off >>= 1) {
+    qm31 o;
+#pragma unroll
+    for (int c = 0; c < 4; c++) o.v[c] = (uint32_t)__shfl_xor((int)top.v[c], off, 64);
+    top = qm_mul_lazy(top, o);
   }
-  const uint32_t per = hpw << kl;
-  for (uint32_t idx = t; idx < per; idx += GKR_THREADS) {
-    const uint4 h = hi[idx >> kl], e = lo[idx & ((1u << kl) - 1)];
-    const qm31 o = qm_mul_lazy({{h.x, h.y, h.z, h.w}}, {{e.x, e.y, e.z, e.w}});
-    if (a16) stqe<true>(buf, (H0 << kl) + idx, o);
-    else stqe<false>(buf, (H0 << kl) + idx, o);
+  if (t < 1u << hb) {  // the first wavefront, lanes below 32 and their mirror: top is its lower half's product
+    qm31 h;
+#pragma unroll
+    for (int c = 0; c < 4; c++) h.v[c] = (uint32_t)__builtin_amdgcn_readfirstlane((int)top.v[c]);
+    h = qm_mul_lazy(h, vq);
+    for (uint32_t i = 0; i < hb; i++) h = qm_mul_lazy(h, eq_factor(ys, k, kl + i, (t >> i) & 1u));
+    hi[t] = make_uint4(h.v[0], h.v[1], h.v[2], h.v[3]);
+  }
+  qm31 lo = one;
+  for (uint32_t i = 0; i < kl; i++) lo = qm_mul_lazy(lo, eq_factor(ys, k, i, (t >> i) & 1u));
+  __syncthreads();
+  if (t >= 1u << kl) return;
+  const uint64_t H0 = (uint64_t)blockIdx.x << hb;
+  for (uint32_t h = 0; h < 1u << hb; h++) {
+    const uint4 x = hi[h];
+    const qm31 o = qm_mul_lazy({{x.x, x.y, x.z, x.w}}, lo);
+    const uint64_t at = ((H0 + h) << kl) + t;
+    if (a16) stqe<true>(buf, at, o);
+    else stqe<false>(buf, at, o);
   }
 }
 
@@ -355,9 +366,10 @@ void gkr_gen_eq_evals(uint32_t* buf, const uint32_t* y, uint32_t k, const uint32
   require(buf && v && (k == 0 || y), "gkr_gen_eq_evals: null pointer");
   require(k <= 31, "gkr_gen_eq_evals: at most 31 variables");
   const uint32_t kl = k < GKR_EQ_LO_MAX ? k : GKR_EQ_LO_MAX;
-  const uint64_t n_hi = 1ull << (k - kl);
-  const uint32_t hpw = (uint32_t)(n_hi < GKR_EQ_HPW ? n_hi : GKR_EQ_HPW);
-  hipLaunchKernelGGL(k_gkr_eq_table, dim3((uint32_t)(n_hi / hpw)), dim3(GKR_THREADS), 0, s, buf, y, k, kl, hpw, v,
+  // entries per lane: as many as leave 256 workgroups, one per CU (at k <= 16
+  // one, where the serial products count), and at most 64
+  const uint32_t rest = k - kl, hb = rest <= 8 ? 0 : rest - 8 < GKR_EQ_HB_MAX ? rest - 8 : GKR_EQ_HB_MAX;
+  hipLaunchKernelGGL(k_gkr_eq_table, dim3(1u << (rest - hb)), dim3(GKR_THREADS), 0, s, buf, y, k, kl, hb, v,
                      al16(buf));
   VX_HIP(hipGetLastError());
 }
