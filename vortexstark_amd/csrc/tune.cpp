@@ -86,9 +86,12 @@ void append_line(const std::string& file, const Key& k, const TreeShape& s) {
 constexpr float MIN_GAIN = 0.03f;
 // A commitment of tens of microseconds is about as long as an event's own
 // jitter: after a single timed run one small tree in three kept a shape that
-// takes 28 us where the built-in one takes 20. The least of five is stable.
+// takes 28 us where the built-in one takes 20. The least of five is stable. A
+// candidate that starts out slower than the best so far by HOPELESS is not run
+// again (it can only lose by that; the built-in shape always gets its runs).
 constexpr float SHORT_MS = 0.2f;
 constexpr int SHORT_REPS = 6;
+constexpr float HOPELESS = 1.25f;
 
 TreeShape measure(const LeafSrc& L, const TreeLevels& T, uint32_t store_lo, hipStream_t s,
                   const std::vector<TreeShape>& cands, const TreeShape& dflt) {
@@ -99,8 +102,12 @@ TreeShape measure(const LeafSrc& L, const TreeLevels& T, uint32_t store_lo, hipS
   float best_ms = 1e30f, dflt_ms = 1e30f;
   try {
     for (const TreeShape& c : cands) {
+      const bool is_dflt = c.tile_log == dflt.tile_log && c.lpt == dflt.lpt;
       float ms = 1e30f;
-      for (int rep = 0; rep < 2 || (rep < SHORT_REPS && ms < SHORT_MS); rep++) {
+      auto again = [&](int rep) {
+        return rep < 2 || (rep < SHORT_REPS && ms < SHORT_MS && (is_dflt || ms < HOPELESS * best_ms));
+      };
+      for (int rep = 0; again(rep); rep++) {
         float one = 0;
         VX_HIP(hipEventRecord(e0, s));
         merkle_commit_shaped(L, T, store_lo, RootHook{}, s, c);
@@ -109,7 +116,7 @@ TreeShape measure(const LeafSrc& L, const TreeLevels& T, uint32_t store_lo, hipS
         VX_HIP(hipEventElapsedTime(&one, e0, e1));
         if (rep > 0) ms = one < ms ? one : ms;  // the first run warms up
       }
-      if (c.tile_log == dflt.tile_log && c.lpt == dflt.lpt) dflt_ms = ms;
+      if (is_dflt) dflt_ms = ms;
       if (ms < best_ms) {
         best_ms = ms;
         best = c;
