@@ -1,5 +1,5 @@
 """The one-launch eq table where its split over lanes, values per lane and
-workgroups changes: 2^8 lanes, one value per lane up to 2^16 entries, 64 from
+workgroups changes: 2^8 lanes, one value per lane up to 2^17 entries, 32 from
 2^22, with extreme coordinates. Against the oracle."""
 import numpy as np
 import pytest

@@ -102,9 +102,9 @@ __global__ __launch_bounds__(GKR_THREADS) void k_gkr_eq_pass(uint32_t* buf, cons
 // store. Field products are exact, so the entries equal the pass-by-pass ones.
 // Serial products bind it up to about 2^20 entries: 2^20 took 24 us with
 // a table of 2^10 low factors built in LDS by ten passes with a barrier each
-// in 64 workgroups, 11.7 us so (3.3 for the stores alone).
+// in 64 workgroups, 11 us so (3.3 for the stores alone).
 constexpr uint32_t GKR_EQ_LO_MAX = 8;  // 2^8 lanes
-constexpr uint32_t GKR_EQ_HB_MAX = 6;
+constexpr uint32_t GKR_EQ_HB_MAX = 5;
 __device__ __forceinline__ qm31 eq_factor(const uint4* y, uint32_t k, uint32_t i, bool bit) {
   const uint4 w = y[k - 1 - i];
   const qm31 yi{{w.x, w.y, w.z, w.w}};
@@ -366,9 +366,10 @@ void gkr_gen_eq_evals(uint32_t* buf, const uint32_t* y, uint32_t k, const uint32
   require(buf && v && (k == 0 || y), "gkr_gen_eq_evals: null pointer");
   require(k <= 31, "gkr_gen_eq_evals: at most 31 variables");
   const uint32_t kl = k < GKR_EQ_LO_MAX ? k : GKR_EQ_LO_MAX;
-  // entries per lane: as many as leave 256 workgroups, one per CU (at k <= 16
-  // one, where the serial products count), and at most 64
-  const uint32_t rest = k - kl, hb = rest <= 8 ? 0 : rest - 8 < GKR_EQ_HB_MAX ? rest - 8 : GKR_EQ_HB_MAX;
+  // entries per lane: as many as leave 512 workgroups, two per CU (2^21
+  // entries: 14 us, with 256 workgroups 17), and at most 32 (2^22: 19 us, with
+  // 64 and 256 workgroups 26; from 2^23 on 16, 32 and 64 are alike)
+  const uint32_t rest = k - kl, hb = rest <= 9 ? 0 : rest - 9 < GKR_EQ_HB_MAX ? rest - 9 : GKR_EQ_HB_MAX;
   hipLaunchKernelGGL(k_gkr_eq_table, dim3(1u << (rest - hb)), dim3(GKR_THREADS), 0, s, buf, y, k, kl, hb, v,
                      al16(buf));
   VX_HIP(hipGetLastError());
