@@ -609,8 +609,8 @@ int vx_bit_reverse_m31_batch(const uint32_t *const *h_src, uint32_t *const *h_ds
  * cuda/merkle_leaves_lifted.cu): leaf i of a 2^lifting_log_size tree =
  * Blake2s of every column's value at its lifted row
  * ((i >> (S - L + 1)) << 1 | (i & 1) for a column of log size L < S), columns
- * sorted by ascending size. The schedule of same-size chunks is derived from
- * h_log_sizes. d_hashes: 8 words per leaf. */
+ * sorted by ascending size, lifting_log_size 2..31. The schedule of same-size
+ * chunks is derived from h_log_sizes. d_hashes: 8 words per leaf. */
 int vx_build_leaves_lifted(const uint32_t *const *h_cols, const uint32_t *h_log_sizes, uint32_t n_cols,
                            uint32_t lifting_log_size, uint32_t *d_hashes, vx_stream_t stream);
 /* Root of that lifted tree (lifting size = the largest column), nodes

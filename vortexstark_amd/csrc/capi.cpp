@@ -1402,7 +1402,7 @@ int vx_bit_reverse_m31_batch(const uint32_t* const* h_src, uint32_t* const* h_ds
 
 static std::vector<LiftCol> lifted_cols(const uint32_t* const* h_cols, const uint32_t* h_log_sizes, uint32_t n_cols,
                                         uint32_t lifting_log) {
-  require(h_cols && h_log_sizes && n_cols >= 1 && lifting_log >= 1 && lifting_log <= 31, "lifted: bad arguments");
+  require(h_cols && h_log_sizes && n_cols >= 1 && lifting_log >= 2 && lifting_log <= 31, "lifted: bad arguments");
   std::vector<LiftCol> lc(n_cols);
   for (uint32_t c = 0; c < n_cols; c++) {
     require(h_cols[c] && h_log_sizes[c] >= 1 && h_log_sizes[c] <= lifting_log, "lifted: column larger than the tree");
