@@ -1171,9 +1171,13 @@ void fri_tail(const FriTailArgs& a, hipStream_t s) {
   uint32_t prev = 0;
   for (uint32_t li = 0; li < a.n_layers; li++) {
     const FriTailLayer& T = a.layer[li];
-    require(T.log_n >= 1 && T.log_n <= TAIL_MAX_LOG && T.lo <= T.log_n && T.tw && T.tree && T.root_out && T.alpha,
+    // levels are stored as they are merged, so from level 1 up
+    require(T.log_n >= 1 && T.log_n <= TAIL_MAX_LOG && T.lo >= 1 && T.lo <= T.log_n && T.tw && T.tree && T.root_out &&
+                T.alpha,
             "fri_tail: bad layer");
     require(li == 0 || T.log_n + 1 == prev, "fri_tail: layers must halve");
+    // only the first layer's challenge is read from memory
+    require(li == 0 || a.layer[li - 1].next_alpha == T.alpha, "fri_tail: a layer folds by what the one before draws");
     for (uint32_t l = T.lo; l < T.log_n; l++)
       require(T.off[l + 1] == T.off[l] + (8u << (T.log_n - l)), "fri_tail: tree levels must lie back to back");
     for (int c = 0; c < 4; c++) require(T.out[c] != nullptr && (li > 0 || a.in[c] != nullptr), "fri_tail: null column");

@@ -338,10 +338,10 @@ constexpr uint32_t TAIL_MAX_LAYERS = TAIL_MAX_LOG;
 struct FriTailLayer {
   uint32_t* out[4];            // layer values (SoA), 2^log_n each
   const uint32_t* tw;          // fold twiddles of the fold that produces this layer
-  uint32_t* tree;              // stored tree levels [lo, log_n]
+  uint32_t* tree;              // stored tree levels [lo, log_n], lo >= 1
   uint32_t off[TAIL_MAX_LOG + 1];
   uint32_t* root_out;          // proof slot of the root
-  const uint32_t* alpha;       // device QM31 used by this fold
+  const uint32_t* alpha;       // device QM31 used by this fold: the next_alpha of the layer before
   uint32_t* next_alpha;        // where to draw the next fold's alpha (null: none)
   uint32_t log_n, lo;
 };
