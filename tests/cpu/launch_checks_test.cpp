@@ -57,6 +57,10 @@ int main(int argc, char** argv) {
   } else if (!std::strcmp(what, "tail_no_challenge")) {
     a.layer[0].next_alpha = nullptr;
     ok = refused([&] { fri_tail(a, nullptr); });
+  } else if (!std::strcmp(what, "proof_destination")) {  // stored 16 bytes at a time
+    ok = refused([&] { set_inputs(word(0x1000), word(0x2000), 3, 1, 1, word(0x3008), nullptr); });
+  } else if (!std::strcmp(what, "inputs_pointer_slot")) {
+    ok = refused([&] { set_inputs(word(0x1004), word(0x2000), 3, 1, 1, word(0x3010), nullptr); });
   }
   std::printf("%s %s\n", ok ? "PASS" : "FAIL", what);
   return ok ? 0 : 1;

@@ -9,7 +9,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "vortexstark_amd")
 
-CASES = ["tail_level_0", "tail_other_challenge", "tail_no_challenge"]
+CASES = ["tail_level_0", "tail_other_challenge", "tail_no_challenge", "proof_destination", "inputs_pointer_slot"]
 
 
 @pytest.fixture(scope="module")

@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256) void k_copy_to_host(uint32_t* const* dst_p, co
 }
 
 void copy_to_host(uint32_t* const* d_dst, const uint32_t* dev_src, uint64_t words, hipStream_t s) {
-  require((reinterpret_cast<uintptr_t>(dev_src) & 15u) == 0, "copy_to_host: 16-byte aligned buffers");
+  require((reinterpret_cast<uintptr_t>(dev_src) & 15u) == 0, "copy_to_host: 16-byte aligned source");
   const uint64_t blocks = ((words >> 2) + 255) / 256;
   const uint32_t grid = (uint32_t)(blocks < 1 ? 1 : (blocks > 512 ? 512 : blocks));
   hipLaunchKernelGGL(k_copy_to_host, dim3(grid), dim3(256), 0, s, d_dst, dev_src, words);

@@ -93,6 +93,9 @@ __global__ void k_set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a,
 
 void set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b, uint32_t* host_dst,
                 hipStream_t s) {
+  // the copy stores 16 bytes per lane and takes the destination from inputs[2..3] as one pointer
+  require((reinterpret_cast<uintptr_t>(host_dst) & 15u) == 0, "set_inputs: 16-byte aligned destination");
+  require((reinterpret_cast<uintptr_t>(inputs) & 7u) == 0, "set_inputs: 8-byte aligned inputs");
   hipLaunchKernelGGL(k_set_inputs, dim3(1), dim3(64), 0, s, inputs, proof, word_a, a, b, host_dst);
   VX_HIP(hipGetLastError());
 }

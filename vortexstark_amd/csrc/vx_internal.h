@@ -227,6 +227,8 @@ void stwo_twiddles(uint32_t log_n, uint32_t* tw, uint32_t* itw, hipStream_t s);
 // ------------------------------------------------- misc kernels (fri.hip)
 void fib_trace(uint32_t a, uint32_t b, uint32_t* out, uint32_t log_n, hipStream_t s);
 void fib_trace_dev(const uint32_t* ab, uint32_t* out, uint32_t log_n, hipStream_t s);
+// inputs[0..1] = (a, b), also into the proof at word_a; inputs[2..3] = host_dst,
+// for copy_to_host.
 void set_inputs(uint32_t* inputs, uint32_t* proof, uint32_t word_a, uint32_t a, uint32_t b, uint32_t* host_dst,
                 hipStream_t s);
 void fib_quotient(const uint32_t* trace, uint32_t* o0, uint32_t* o1, uint32_t* o2, uint32_t* o3,
@@ -479,8 +481,10 @@ void poseidon_grind_min(const uint64_t* d_prefix_mont, uint32_t pow_bits, uint64
 void poseidon_leaves(const uint32_t* const* d_cols, const uint32_t* d_logs, uint32_t n_cols, uint32_t lifting_log,
                      uint64_t* d_out, uint32_t n_leaves, hipStream_t s);
 void poseidon_next_layer(const uint64_t* d_prev, uint64_t* d_out, uint32_t n_parents, hipStream_t s);
-// Copy `words` words from device memory into pinned host memory
-// (hipHostMalloc) with a kernel; both 16-byte aligned.
+// Copy `words` words from device memory (16-byte aligned) into pinned host
+// memory (hipHostMalloc) with a kernel. d_dst is in device memory and holds the
+// destination as the device addresses it when the kernel runs; set_inputs puts
+// it there and checks that it is 16-byte aligned.
 void copy_to_host(uint32_t* const* d_dst, const uint32_t* dev_src, uint64_t words, hipStream_t s);
 
 // ------------------------------------- synthetic multi-column AIR (d2.hip)
