@@ -108,8 +108,6 @@ class StarkProver {
   }
   // One eager proof of dummy inputs: every merkle_commit of this class is
   // timed by the autotuner (if enabled) before a graph freezes the shapes.
-  void write_header();
-  void put_inputs(uint32_t a, uint32_t b, uint32_t buffer);
   void tune();
   bool graphs() const { return use_graph_; }
   // Device bytes a prover of this class allocates for itself (tables excluded).
@@ -129,6 +127,10 @@ class StarkProver {
  private:
   void build_descs();
   void build_batch();
+  void write_header();
+  // Enqueued on the prover's stream, so the proofs before it have been copied
+  // to their own buffer by then.
+  void put_inputs(uint32_t a, uint32_t b, uint32_t buffer);
   void record(bool timed, hipStream_t s);
   void capture();
   TreeLevels tree_levels(uint32_t idx) const;
