@@ -271,6 +271,19 @@ void grind_pow_batch(const uint32_t* d_prefix, uint64_t* d_result, uint32_t pow_
   launch_grind<false>(grid, m31_out, d_prefix, pow_bits, best, batch_offset, n, s);
 }
 
+__global__ void k_write_words(uint32_t* dst, WordWrites w) {
+  if (threadIdx.x < w.n) dst[w.at[threadIdx.x]] = w.value[threadIdx.x];
+}
+
+// A few words at scattered places by one launch. (Four or five synchronous
+// copies from pageable memory in its place made creating a prover slower: at
+// log_n = 12 437 us against 384, at 20 1,824 against 1,218.)
+void write_words(uint32_t* dst, const WordWrites& w, hipStream_t s) {
+  if (w.n == 0) return;
+  hipLaunchKernelGGL(k_write_words, dim3(1), dim3(64), 0, s, dst, w);
+  VX_HIP(hipGetLastError());
+}
+
 // Proof download by the GPU itself: the workgroups store the proof
 // straight into pinned host memory (mapped into the device's address space),
 // 16 bytes per lane per step, instead of a DMA copy whose start-up cost

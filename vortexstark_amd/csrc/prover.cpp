@@ -308,11 +308,12 @@ StarkProver::StarkProver(uint32_t log_n, uint32_t blowup_bits, uint32_t n_querie
   build_descs();
 }
 
-// The proof words that every proof of this prover has alike.
+// The proof words that every proof of this prover has alike, by one launch on
+// the prover's stream: no proof waits for it, nor does the constructor.
 void StarkProver::write_header() {
-  const ProofLayout& L = layout_;
-  auto put = [&](uint64_t word, const std::vector<uint32_t>& v) {
-    VX_HIP(hipMemcpy(proof_.u32() + word, v.data(), 4 * v.size(), hipMemcpyHostToDevice));
+  WordWrites w{};
+  auto put = [&](uint64_t word, std::initializer_list<uint32_t> v) {
+    for (uint32_t x : v) w.add((uint32_t)word++, x);
   };
   if (air_.kind == AIR_FIBONACCI) {  // words 3, 4 (a, b) are written by set_inputs
     put(0, {KRAK_MAGIC, pow_bits_ ? 2u : 1u, log_n_});
@@ -321,8 +322,9 @@ void StarkProver::write_header() {
     put(0, {KRAK_MAGIC, 3, log_n_, air_.n_cols, air_.n_cons, blowup_, pow_bits_, 0, 0});
     put(11, {(uint32_t)air_.air_seed, (uint32_t)(air_.air_seed >> 32), n_groups_});
   }
-  put(L.w_nfri, {n_fri_});
-  put(L.w_nfdec, {n_fri_});
+  put(layout_.w_nfri, {n_fri_});
+  put(layout_.w_nfdec, {n_fri_});
+  write_words(proof_.u32(), w, stream_);
 }
 
 // Work lists, lifted column table, column offsets and the constant header

@@ -481,6 +481,18 @@ void poseidon_grind_min(const uint64_t* d_prefix_mont, uint32_t pow_bits, uint64
 void poseidon_leaves(const uint32_t* const* d_cols, const uint32_t* d_logs, uint32_t n_cols, uint32_t lifting_log,
                      uint64_t* d_out, uint32_t n_leaves, hipStream_t s);
 void poseidon_next_layer(const uint64_t* d_prev, uint64_t* d_out, uint32_t n_parents, hipStream_t s);
+// dst[at] = value for up to MAX words, asynchronously.
+struct WordWrites {
+  static constexpr uint32_t MAX = 16;
+  uint32_t n;
+  uint32_t at[MAX], value[MAX];
+  void add(uint32_t where, uint32_t what) {
+    require(n < MAX, "write_words: at most 16 words");
+    at[n] = where;
+    value[n++] = what;
+  }
+};
+void write_words(uint32_t* dst, const WordWrites& w, hipStream_t s);
 // Copy `words` words from device memory (16-byte aligned) into pinned host
 // memory (hipHostMalloc) with a kernel. d_dst is in device memory and holds the
 // destination as the device addresses it when the kernel runs; set_inputs puts
