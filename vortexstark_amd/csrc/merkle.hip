@@ -861,8 +861,9 @@ static uint32_t lane_log_for(uint32_t tile_log) {
 
 // Two wavefronts per SIMD (512 workgroups of 256 lanes on 256 CUs) is where
 // b2_compress_wide overtakes b2_compress: 33 -> 40 giga-compressions/s there,
-// 31 -> 24 with one. Shapes of 8 and 16 leaves per lane are for trees whose
-// grids are larger, so they have only that form.
+// 31 -> 24 with one. That holds for every shape (one column, 16 leaves per lane:
+// 256 workgroups 97 us wide and 72 not, 512 workgroups 104 wide; 8 leaves per
+// lane: 256 workgroups 58 and 46, 512 workgroups 63 wide).
 static bool wide_grid(uint64_t workgroups) { return workgroups >= 512; }
 
 template <uint32_t KIND, uint32_t NC, uint32_t LPT>
@@ -872,11 +873,11 @@ static void launch_subtree_lpt(const LeafSrc& L, const TreeLevels& T, uint32_t t
   if (tile_log == T.log_n)
     hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, true, false>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
                        tile_log, store_lo, hook);
-  else if (LPT >= 3 || wide_grid(grid))
+  else if (wide_grid(grid))
     hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, false, true>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
                        tile_log, store_lo, hook);
   else
-    hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, false, LPT >= 3>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
+    hipLaunchKernelGGL((k_subtree<KIND, NC, LPT, false, false>), dim3((uint32_t)grid), dim3(SUB_THREADS), 0, s, L, T,
                        tile_log, store_lo, hook);
 }
 
