@@ -195,9 +195,9 @@ int vx_eval_at_point(const uint32_t *d_coeffs, const uint32_t *d_folding_factors
  * max_log_n factors (d_folding_factors, the factors of a 2^max_log_n
  * polynomial, as for vx_eval_at_point). h_cols and h_log_sizes are HOST
  * arrays (the reference passes device arrays); columns of 4 or more words
- * 16-byte aligned. d_results: n_cols QM31 (device). One launch for every
- * 2^14-coefficient chunk of every column, then one per fold level.
- * Synchronous. */
+ * 16-byte aligned. d_results: n_cols QM31 (device). Three launches: tables of
+ * the point's weights, the 2^14-coefficient chunks of every column, and the
+ * sum of each column's chunks. Synchronous. */
 int vx_eval_at_point_batch(const uint32_t *const *h_cols, const uint32_t *h_log_sizes, uint32_t n_cols,
                            const uint32_t *d_folding_factors, uint32_t max_log_n, uint32_t *d_results,
                            vx_stream_t stream);

@@ -1,5 +1,5 @@
 """The chunked evaluation of many columns (vx_eval_at_point_batch): more
-columns than one launch takes, sizes around the 2^14-coefficient chunk,
+columns than the kernels' arguments take, sizes around the 2^14-coefficient chunk,
 several chunks per workgroup, and extreme coefficients (0 and P - 1, where
 the 64-bit sums are largest). Field values against the oracle."""
 import ctypes as C

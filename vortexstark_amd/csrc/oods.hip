@@ -15,6 +15,8 @@
 // 16 products of F[0..3] in LDS). Products are accumulated 4 per 64-bit sum
 // before a reduction; a workgroup folds its lanes in LDS, and the block sums
 // are folded 256 at a time with the next 8 factors.
+#include <algorithm>
+
 #include "prover.h"
 #include "vx_internal.h"
 #include "vx_blake2s_x4.h"
@@ -236,17 +238,25 @@ const uint32_t* eval_at_point(const uint32_t* c, const uint32_t* factors, uint32
 // fold; the shift's share of the sum is the constant C). The tree folds of
 // the lanes by QM31 products that this replaces were two thirds of the
 // kernel's instructions. 64 columns of 2^20 at two points (268 MB): 192 -> 51 us
-// (the read at a large copy's rate takes 52); the OODS step 338 -> 133 us.
+// (the read at a large copy's rate takes 52); the OODS step 338 -> 117 us.
 static constexpr uint32_t EV_TERMS = 64;      // coefficients per lane and chunk
 static constexpr uint32_t EV_MAX_WGS = 2048;  // of a call: chunks per workgroup grow beyond
-static constexpr uint32_t EV_ARG_COLS = 192;  // columns per launch (kernel arguments)
+static constexpr uint32_t EV_ARG_COLS = 192;  // columns that travel in the kernels' arguments
 
-struct EvalCols {
-  const uint32_t* col[EV_ARG_COLS];
-  uint32_t first[EV_ARG_COLS];  // workgroup of the column's first chunk, ascending from 0
-  uint8_t log_n[EV_ARG_COLS];
-  uint32_t n, cpw_log, wg_base;  // 2^cpw_log chunks per workgroup; wg_base: workgroups of earlier launches
+struct EvalCol {
+  const uint32_t* p;
+  uint32_t first;  // workgroup of the column's first chunk, ascending from 0
+  uint32_t log_n;
 };
+// The columns are an array in the kernels' own arguments, or, when there are
+// more, a table uploaded into the workspace. (Splitting them over launches of
+// EV_ARG_COLS columns instead took 676 us for 10,000 columns of 2^8, the table
+// takes 114; 500 columns 52 and 33.)
+struct EvalArgs {
+  EvalCol col[EV_ARG_COLS];
+};
+__device__ __forceinline__ EvalCol eval_col(const EvalArgs& cols, uint32_t k) { return cols.col[k]; }
+__device__ __forceinline__ EvalCol eval_col(const EvalCol* cols, uint32_t k) { return ld_uniform(cols + k); }
 // words of the tables of np points, G having 2^g_log entries
 struct EvalTables {
   uint32_t np, g_log;
@@ -314,22 +324,24 @@ __device__ __forceinline__ uint32_t wave_sum_mod_p(uint32_t v) {
   return v;
 }
 
-template <uint32_t NP>
-__global__ __launch_bounds__(EV_WG) void k_eval_chunks(EvalCols a, EvalTables T, const uint32_t* tables,
-                                                       uint32_t* part, uint32_t part_stride) {
+// A workgroup takes 2^cpw_log chunks.
+template <uint32_t NP, typename Cols>
+__global__ __launch_bounds__(EV_WG) void k_eval_chunks(Cols cols, uint32_t n_cols, uint32_t cpw_log, EvalTables T,
+                                                       const uint32_t* tables, uint32_t* part, uint32_t part_stride) {
   __shared__ qm31 red[NP][EV_WG / 64];
   const uint32_t wg = blockIdx.x, t = threadIdx.x;
-  uint32_t lo = 0, hi = a.n;
+  uint32_t lo = 0, hi = n_cols;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (a.first[mid] <= wg) lo = mid;
+    if (eval_col(cols, mid).first <= wg) lo = mid;
     else hi = mid;
   }
-  const uint32_t* col = a.col[lo];
-  const uint32_t L = a.log_n[lo];
+  const EvalCol c = eval_col(cols, lo);
+  const uint32_t* col = c.p;
+  const uint32_t L = c.log_n;
   const uint32_t n = 1u << L;
   const uint32_t chunks = L > EV_BIG_LOG ? 1u << (L - EV_BIG_LOG) : 1u;
-  const uint32_t c0 = (wg - a.first[lo]) << a.cpw_log, c1 = min(c0 + (1u << a.cpw_log), chunks);
+  const uint32_t c0 = (wg - c.first) << cpw_log, c1 = min(c0 + (1u << cpw_log), chunks);
   qm31 sum[NP];
 #pragma unroll
   for (uint32_t pt = 0; pt < NP; pt++) sum[pt] = qm31{{0u, 0u, 0u, 0u}};
@@ -408,18 +420,18 @@ __global__ __launch_bounds__(EV_WG) void k_eval_chunks(EvalCols a, EvalTables T,
   if (t < NP) {
     qm31 s = red[t][0];
     for (uint32_t w = 1; w < EV_WG / 64; w++) s = qm_add(s, red[t][w]);
-    reinterpret_cast<qm31*>(part)[(uint64_t)t * part_stride + a.wg_base + wg] = s;
+    reinterpret_cast<qm31*>(part)[(uint64_t)t * part_stride + wg] = s;
   }
 }
 
-// results[pt * n_cols + col_base + k] = the sum of column k's workgroups'
-// sums; one wavefront per (column, point).
-__global__ __launch_bounds__(64) void k_eval_sum(EvalCols a, uint32_t n_wgs, const uint32_t* part,
-                                                 uint32_t part_stride, uint32_t* results, uint32_t n_cols,
-                                                 uint32_t col_base) {
+// results[pt * n_cols + k] = the sum of column k's workgroups' sums; one
+// wavefront per (column, point).
+template <typename Cols>
+__global__ __launch_bounds__(64) void k_eval_sum(Cols cols, uint32_t n_cols, uint32_t n_wgs, const uint32_t* part,
+                                                 uint32_t* results) {
   const uint32_t k = blockIdx.x, pt = blockIdx.y, lane = threadIdx.x;
-  const uint32_t b = a.first[k], e = k + 1 < a.n ? a.first[k + 1] : n_wgs;
-  const qm31* p = reinterpret_cast<const qm31*>(part) + (uint64_t)pt * part_stride + a.wg_base;
+  const uint32_t b = eval_col(cols, k).first, e = k + 1 < n_cols ? eval_col(cols, k + 1).first : n_wgs;
+  const qm31* p = reinterpret_cast<const qm31*>(part) + (uint64_t)pt * n_wgs;
   uint64_t s[4] = {0, 0, 0, 0};
   for (uint32_t i = b + lane; i < e; i += 64)
 #pragma unroll
@@ -427,16 +439,19 @@ __global__ __launch_bounds__(64) void k_eval_sum(EvalCols a, uint32_t n_wgs, con
 #pragma unroll
   for (int c = 0; c < 4; c++) {
     const uint32_t v = wave_sum_mod_p(m31_reduce64(s[c]));
-    if (lane == 0) results[4 * ((uint64_t)pt * n_cols + col_base + k) + c] = v;
+    if (lane == 0) results[4 * ((uint64_t)pt * n_cols + k) + c] = v;
   }
 }
 
 // The split of a batch into workgroups and its workspace, after checking it.
 struct EvalPlan {
-  EvalTables T;
-  uint32_t cpw_log;
-  uint64_t wgs;
-  uint64_t ws_words() const { return T.words() + 4ull * T.np * wgs; }
+  EvalTables T{};
+  uint32_t cpw_log = 0;
+  uint32_t wgs = 0;
+  std::vector<EvalCol> cols;
+  uint64_t part_words() const { return 4ull * T.np * wgs; }
+  uint64_t col_words() const { return cols.size() > EV_ARG_COLS ? cols.size() * (sizeof(EvalCol) / 4) : 0; }
+  uint64_t ws_words() const { return T.words() + part_words() + col_words(); }
 };
 static uint32_t eval_wgs_of(uint32_t L, uint32_t cpw_log) {
   const uint32_t c = L > EV_BIG_LOG ? L - EV_BIG_LOG : 0;
@@ -461,47 +476,49 @@ static EvalPlan eval_plan(const uint32_t* const* h_cols, const uint32_t* h_log_s
   // once per workgroup, so no more workgroups than keep the chip full.
   uint32_t cpw_log = 0;
   while ((total >> cpw_log) > EV_MAX_WGS) cpw_log++;
-  uint64_t wgs = 0;
-  for (uint32_t k = 0; k < n_cols; k++) wgs += eval_wgs_of(h_log_sizes[k], cpw_log);
-  return {EvalTables{np, top > EV_BIG_LOG ? top - EV_BIG_LOG : 0}, cpw_log, wgs};
+  EvalPlan plan;
+  plan.T = EvalTables{np, top > EV_BIG_LOG ? top - EV_BIG_LOG : 0};
+  plan.cpw_log = cpw_log;
+  plan.cols.resize(n_cols);
+  for (uint32_t k = 0; k < n_cols; k++) {
+    plan.cols[k] = {h_cols[k], plan.wgs, h_log_sizes[k]};
+    plan.wgs += eval_wgs_of(h_log_sizes[k], cpw_log);
+  }
+  return plan;
+}
+
+template <typename Cols>
+static void eval_launch(const EvalPlan& plan, const Cols& cols, const uint32_t* tables, uint32_t* part,
+                        uint32_t* results, hipStream_t s) {
+  const uint32_t n = (uint32_t)plan.cols.size();
+  hipLaunchKernelGGL((plan.T.np == 2 ? k_eval_chunks<2, Cols> : k_eval_chunks<1, Cols>), dim3(plan.wgs), dim3(EV_WG), 0,
+                     s, cols, n, plan.cpw_log, plan.T, tables, part, plan.wgs);
+  VX_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_eval_sum<Cols>, dim3(n, plan.T.np), dim3(64), 0, s, cols, n, plan.wgs, part, results);
+  VX_HIP(hipGetLastError());
 }
 
 // np points (1 or 2): factors holds np tables of 4 max_log_n words back to
-// back (4 words when max_log_n is 0), results np arrays of n_cols QM31.
-// The work is enqueued on s; the workspace (ws_words) must outlive it.
-static void eval_batch_points(const EvalPlan& plan, const uint32_t* const* h_cols, const uint32_t* h_log_sizes,
-                              uint32_t n_cols, const uint32_t* factors, uint32_t max_log_n, uint32_t* results,
+// back (4 words when max_log_n is 0), results np arrays of n_cols QM31. The
+// work is enqueued on s; the plan and the workspace (ws_words) must outlive it.
+static void eval_batch_points(const EvalPlan& plan, const uint32_t* factors, uint32_t max_log_n, uint32_t* results,
                               uint32_t* ws, hipStream_t s) {
   const EvalTables& T = plan.T;
-  const uint32_t np = T.np, cpw_log = plan.cpw_log;
-  const uint64_t wgs = plan.wgs;
+  const uint32_t n_cols = (uint32_t)plan.cols.size();
   uint32_t* tables = ws;
   uint32_t* part = tables + T.words();
   const uint64_t entries = EV_TERMS + 1 + EV_WG + (1ull << T.g_log);
-  hipLaunchKernelGGL(k_eval_tables, dim3((uint32_t)((entries + EV_WG - 1) / EV_WG), np), dim3(EV_WG), 0, s, factors,
+  hipLaunchKernelGGL(k_eval_tables, dim3((uint32_t)((entries + EV_WG - 1) / EV_WG), T.np), dim3(EV_WG), 0, s, factors,
                      max_log_n, T, tables);
   VX_HIP(hipGetLastError());
-  uint32_t wg_base = 0;
-  for (uint32_t k0 = 0; k0 < n_cols; k0 += EV_ARG_COLS) {
-    EvalCols a{};
-    a.n = n_cols - k0 < EV_ARG_COLS ? n_cols - k0 : EV_ARG_COLS;
-    a.cpw_log = cpw_log;
-    a.wg_base = wg_base;
-    uint32_t w = 0;
-    for (uint32_t k = 0; k < a.n; k++) {
-      a.col[k] = h_cols[k0 + k];
-      a.log_n[k] = (uint8_t)h_log_sizes[k0 + k];
-      a.first[k] = w;
-      w += eval_wgs_of(h_log_sizes[k0 + k], cpw_log);
-    }
-    if (np == 2)
-      hipLaunchKernelGGL(k_eval_chunks<2>, dim3(w), dim3(EV_WG), 0, s, a, T, tables, part, (uint32_t)wgs);
-    else
-      hipLaunchKernelGGL(k_eval_chunks<1>, dim3(w), dim3(EV_WG), 0, s, a, T, tables, part, (uint32_t)wgs);
-    VX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_eval_sum, dim3(a.n, np), dim3(64), 0, s, a, w, part, (uint32_t)wgs, results, n_cols, k0);
-    VX_HIP(hipGetLastError());
-    wg_base += w;
+  if (n_cols <= EV_ARG_COLS) {
+    EvalArgs a{};
+    std::copy(plan.cols.begin(), plan.cols.end(), a.col);
+    eval_launch(plan, a, tables, part, results, s);
+  } else {
+    EvalCol* table = reinterpret_cast<EvalCol*>(part + plan.part_words());
+    VX_HIP(hipMemcpyAsync(table, plan.cols.data(), sizeof(EvalCol) * n_cols, hipMemcpyHostToDevice, s));
+    eval_launch(plan, static_cast<const EvalCol*>(table), tables, part, results, s);
   }
 }
 
@@ -510,7 +527,7 @@ void eval_at_point_batch(const uint32_t* const* h_cols, const uint32_t* h_log_si
   if (n_cols == 0) return;
   const EvalPlan plan = eval_plan(h_cols, h_log_sizes, n_cols, 1, max_log_n);
   DeviceBuf ws(4 * plan.ws_words());
-  eval_batch_points(plan, h_cols, h_log_sizes, n_cols, factors, max_log_n, results, ws.u32(), s);
+  eval_batch_points(plan, factors, max_log_n, results, ws.u32(), s);
   VX_HIP(hipStreamSynchronize(s));  // the workspace is freed on return
 }
 
@@ -689,7 +706,7 @@ void oods_sample(uint32_t* d_channel, const uint32_t* const* h_cols, const uint3
   for (uint32_t k = 0; k < n_cols; k++) max_log = h_log_sizes[k] > max_log ? h_log_sizes[k] : max_log;
   const uint32_t fw = 4 * (max_log ? max_log : 1);
   // one allocation: both points' factors, then the evaluation's workspace
-  EvalPlan plan{};
+  EvalPlan plan;
   if (n_cols) plan = eval_plan(h_cols, h_log_sizes, n_cols, 2, max_log);
   const uint64_t ws_at = (2ull * fw + 63) & ~63ull;
   DeviceBuf buf(4 * (ws_at + (n_cols ? plan.ws_words() : 0)));
@@ -698,7 +715,7 @@ void oods_sample(uint32_t* d_channel, const uint32_t* const* h_cols, const uint3
   VX_HIP(hipGetLastError());
   if (n_cols) {
     // both points from one read of every column: values at z, then at z_next
-    eval_batch_points(plan, h_cols, h_log_sizes, n_cols, fz, max_log, d_values, buf.u32() + ws_at, s);
+    eval_batch_points(plan, fz, max_log, d_values, buf.u32() + ws_at, s);
     hipLaunchKernelGGL(k_oods_mix, dim3(1), dim3(MIX_THREADS), 0, s, d_channel, d_values, 2 * n_cols);
     VX_HIP(hipGetLastError());
   }
