@@ -85,11 +85,13 @@ static void ntt_cols(uint32_t* const* dst, const uint32_t* const* src, uint32_t 
   constexpr uint32_t CHUNK = 65535;
   const uint32_t m0 = n_cols < CHUNK ? n_cols : CHUNK;
   DeviceBuf d((src ? 2 : 1) * sizeof(uint32_t*) * (size_t)m0);
+  std::vector<const uint32_t*> both;  // destinations, then sources: one upload (two: 300 columns of 2^8 23.2 us, not 20.2)
   for (uint32_t c0 = 0; c0 < n_cols; c0 += CHUNK) {
     const uint32_t m = n_cols - c0 < CHUNK ? n_cols - c0 : CHUNK;
     uint32_t** dc = static_cast<uint32_t**>(d.p);
-    VX_HIP(hipMemcpyAsync(dc, dst + c0, sizeof(uint32_t*) * m, hipMemcpyHostToDevice, s));
-    if (src) VX_HIP(hipMemcpyAsync(dc + m, src + c0, sizeof(uint32_t*) * m, hipMemcpyHostToDevice, s));
+    both.assign(dst + c0, dst + c0 + m);
+    if (src) both.insert(both.end(), src + c0, src + c0 + m);
+    VX_HIP(hipMemcpyAsync(dc, both.data(), sizeof(uint32_t*) * both.size(), hipMemcpyHostToDevice, s));
     f(NttCols{dc, src ? const_cast<const uint32_t* const*>(dc + m) : nullptr, m, true});
     VX_HIP(hipStreamSynchronize(s));
   }
