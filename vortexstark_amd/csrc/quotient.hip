@@ -17,9 +17,10 @@
 //   den_j(d) = (Re p.x - d.x) Im p.y - (Re p.y - d.y) Im p.x    (CM31),
 // dividing each CM31 half of the QM31 numerator. The reference inverts every
 // den_j(d) with its own Fermat power (about 60 multiplications). Here a lane
-// takes 8 rows (coalesced, 256 apart) and inverts the 8 norms of each
-// accumulator with one Fermat power (Montgomery's trick; a zero norm maps to
-// zero, as the reference's inverse does), so the inversions cost an eighth.
+// takes 8 rows (coalesced, 256 apart; one where the rows are few) and inverts
+// the 8 norms of each accumulator with one Fermat power (Montgomery's trick; a
+// zero norm maps to zero, as the reference's inverse does), so the inversions
+// cost an eighth.
 // Products are summed in 64 bits and reduced once per output (23 products and
 // 16 reductions per row and accumulator), and the numerators are loaded before
 // the inversion, a serial chain of about 45 products. Two accumulators of 2^20
@@ -185,8 +186,14 @@ void accumulate_numerators(const uint32_t* const* cols, const uint32_t* idx_z, c
 }
 
 // ---------------------------------------------------------------------------
-static constexpr uint32_t QC_ROWS = 8;  // rows per lane, QC_THREADS apart
 static constexpr uint32_t QC_THREADS = 256;
+static constexpr uint32_t QC_ROWS = 8;  // rows per lane, QC_THREADS apart
+// Up to two workgroups per CU with one row per lane there is room to run them
+// all at once, and eight rows per lane are a longer chain, most of it for rows
+// past the end when there are few. Two accumulators, eight rows / one row per
+// lane: 2^8 rows 10.9 / 6.1 us, 2^17 11.8 / 7.7, 2^18 12.1 / 11.0 (five: 26.0 /
+// 24.2), 2^19 12.6 / 17.9.
+static constexpr uint32_t QC_FEW = 512 * QC_THREADS;
 
 struct QcArgs {
   const uint32_t* sp_x;
@@ -201,12 +208,13 @@ struct QcArgs {
   uint32_t* out[4];
 };
 
+template <uint32_t ROWS>
 __global__ __launch_bounds__(QC_THREADS) void k_quotients_combine(QcArgs a) {
-  const uint32_t base = blockIdx.x * (QC_THREADS * QC_ROWS) + threadIdx.x;
-  uint32_t dx[QC_ROWS], dy[QC_ROWS];
-  qm31 q[QC_ROWS];
+  const uint32_t base = blockIdx.x * (QC_THREADS * ROWS) + threadIdx.x;
+  uint32_t dx[ROWS], dy[ROWS];
+  qm31 q[ROWS];
 #pragma unroll
-  for (uint32_t r = 0; r < QC_ROWS; r++) {
+  for (uint32_t r = 0; r < ROWS; r++) {
     const uint32_t row = base + r * QC_THREADS;
     const uint32_t at = min(row, a.n_rows - 1);  // past the end: the last row once more, not stored
     dx[r] = as_global(a.xs)[at];
@@ -229,9 +237,9 @@ __global__ __launch_bounds__(QC_THREADS) void k_quotients_combine(QcArgs a) {
 #pragma unroll
     for (int k = 0; k < 4; k++) np[k] = as_global(ld_uniform(a.numer[k] + j));
     // every row's numerators first: their loads are in flight during the inversion
-    uint32_t nu[QC_ROWS][4];
+    uint32_t nu[ROWS][4];
 #pragma unroll
-    for (uint32_t r = 0; r < QC_ROWS; r++) {
+    for (uint32_t r = 0; r < ROWS; r++) {
       const uint32_t row = min(base + r * QC_THREADS, a.n_rows - 1);
       const uint32_t li = min(((row >> sh) << 1) + (row & 1u), last);
 #pragma unroll
@@ -244,10 +252,10 @@ __global__ __launch_bounds__(QC_THREADS) void k_quotients_combine(QcArgs a) {
     uint64_t nal[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) nal[k] = P - al.v[k];
-    uint32_t den[QC_ROWS][2], nrm[QC_ROWS], pre[QC_ROWS];
+    uint32_t den[ROWS][2], nrm[ROWS], pre[ROWS];
     uint32_t acc = 1;
 #pragma unroll
-    for (uint32_t r = 0; r < QC_ROWS; r++) {
+    for (uint32_t r = 0; r < ROWS; r++) {
       den[r][0] = m31_reduce64((uint64_t)(P - piy.a) * dx[r] + (uint64_t)pix.a * dy[r] + k0.a);
       den[r][1] = m31_reduce64((uint64_t)(P - piy.b) * dx[r] + (uint64_t)pix.b * dy[r] + k0.b);
       nrm[r] = m31_reduce64((uint64_t)den[r][0] * den[r][0] + (uint64_t)den[r][1] * den[r][1]);
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(QC_THREADS) void k_quotients_combine(QcArgs a) {
     }
     uint32_t inv = m31_inv(acc);
 #pragma unroll
-    for (int r = QC_ROWS - 1; r >= 0; r--) {
+    for (int r = ROWS - 1; r >= 0; r--) {
       const uint32_t inv_n = nrm[r] ? m31_reduce64((uint64_t)inv * pre[r]) : 0u;
       inv = m31_reduce64((uint64_t)inv * (nrm[r] ? nrm[r] : 1u));
       // conj / norm = (da, -db); ndb = db is its negative
@@ -273,7 +281,7 @@ __global__ __launch_bounds__(QC_THREADS) void k_quotients_combine(QcArgs a) {
     }
   }
 #pragma unroll
-  for (uint32_t r = 0; r < QC_ROWS; r++) {
+  for (uint32_t r = 0; r < ROWS; r++) {
     const uint32_t row = base + r * QC_THREADS;
     if (row >= a.n_rows) continue;
 #pragma unroll
@@ -288,8 +296,9 @@ void quotients_combine(const uint32_t* sp_x, const uint32_t* sp_y, const uint32_
   if (n_rows == 0) return;
   QcArgs a{sp_x, sp_y, fla, {numer[0], numer[1], numer[2], numer[3]}, acc_log_sizes, n_accs, xs, ys,
            lifting_log_size, n_rows, {out[0], out[1], out[2], out[3]}};
-  const uint32_t per_block = QC_THREADS * QC_ROWS;
-  hipLaunchKernelGGL(k_quotients_combine, dim3((n_rows + per_block - 1) / per_block), dim3(QC_THREADS), 0, s, a);
+  const uint32_t rows = n_rows <= QC_FEW ? 1 : QC_ROWS, per_block = QC_THREADS * rows;
+  hipLaunchKernelGGL(rows == 1 ? k_quotients_combine<1> : k_quotients_combine<QC_ROWS>,
+                     dim3((n_rows + per_block - 1) / per_block), dim3(QC_THREADS), 0, s, a);
   VX_HIP(hipGetLastError());
 }
 
