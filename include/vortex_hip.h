@@ -864,7 +864,9 @@ int vx_fold_line_commit(const uint32_t *i0, const uint32_t *i1, const uint32_t *
  * fastest is cached; all shapes give the same tree, so proofs do not change.
  * Provers run one eager proof before capturing their graph so that every
  * commitment of the class is tuned. enabled = 0 uses the built-in shapes.
- * cache_file (may be NULL): entries are loaded from it and appended to it. */
+ * cache_file (may be NULL): entries are loaded from it and appended to it,
+ * with the revision of the kernels that were timed; entries of another
+ * revision are measured again, lines without one are taken as they are. */
 int vx_tuner_configure(int enabled, const char *cache_file);
 /* Up to `capacity` cached entries, 9 words each: device, leaf kind, n_cols,
  * n_cons, lifted columns, log_n, stored-from level, tile log, leaves-per-lane

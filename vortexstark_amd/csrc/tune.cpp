@@ -8,14 +8,16 @@
 // table, the first commitment of each key (leaf kind, columns, constraints,
 // log_n, stored levels) on a device is timed with every valid shape, twice
 // each (the second run counts; short ones six times, the least counts), on
-// the caller's stream and with the caller's buffers, and the fastest is cached for the process (the built-in
-// shape unless another is more than 3 % faster). All shapes
-// produce the same tree, so the choice never changes a proof. Measuring
-// needs a stream synchronisation, so it never happens while the stream is
-// being captured into a graph (the provers run one eager proof first, see
-// StarkProver::tune). An optional cache file keeps the choices across
-// processes: one line "kind n_cols n_cons lift_n log_n store_lo tile_log lpt"
-// per key.
+// the caller's stream and with the caller's buffers, and the fastest is cached
+// for the process (the built-in shape unless another is more than 3 % faster).
+// All shapes produce the same tree, so the choice never changes a proof.
+// Measuring needs a stream synchronisation, so it never happens while the
+// stream is being captured into a graph (the provers run one eager proof
+// first, see StarkProver::tune). An optional cache file keeps the choices
+// across processes: one line "kind n_cols n_cons lift_n log_n store_lo
+// tile_log lpt" per key, then the revision of the kernels that were timed
+// ("r1"); a line of another revision is not taken, one without (written by
+// hand, to pin a shape) is.
 //
 // The circle NTT is tuned the same way per transform shape (direction,
 // log_n, transformed bits, columns, basis): the built-in plan, tiles in
@@ -23,8 +25,9 @@
 // allow) the strided bits over one more pass, each timed twice on the
 // caller's stream; out-of-place transforms are timed on the caller's
 // buffers, in-place ones on a scratch buffer of the same shape. Cache-file
-// lines "ntt fwd log_n eff_bits n_cols stwo split order".
+// lines "ntt fwd log_n eff_bits n_cols stwo split order", with the revision.
 #include <cstdio>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
@@ -37,6 +40,10 @@
 namespace vx {
 
 namespace {
+
+// Raised with every change to the tree or transform kernels or to how they are
+// timed that can change which choice is the fastest.
+constexpr unsigned REVISION = 1;
 
 using Key = std::tuple<int, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t>;
 
@@ -75,8 +82,8 @@ void append_line(const std::string& file, const Key& k, const TreeShape& s) {
   if (file.empty()) return;
   FILE* f = std::fopen(file.c_str(), "a");
   if (!f) return;  // the cache file is an optimisation: a read-only path only costs re-measuring
-  std::fprintf(f, "%u %u %u %u %u %u %u %u\n", (unsigned)std::get<1>(k), std::get<2>(k), std::get<3>(k),
-               std::get<4>(k), std::get<5>(k), std::get<6>(k), s.tile_log, s.lpt);
+  std::fprintf(f, "%u %u %u %u %u %u %u %u r%u\n", (unsigned)std::get<1>(k), std::get<2>(k), std::get<3>(k),
+               std::get<4>(k), std::get<5>(k), std::get<6>(k), s.tile_log, s.lpt, REVISION);
   std::fclose(f);
 }
 
@@ -230,8 +237,8 @@ NttPlan tuned_ntt_plan(const NttKey& key, hipStream_t s, const std::function<boo
     t.measured++;
     if (!t.file.empty()) {
       if (FILE* f = std::fopen(t.file.c_str(), "a")) {
-        std::fprintf(f, "ntt %u %u %u %u %u %u %u\n", std::get<1>(k), std::get<2>(k), std::get<3>(k),
-                     std::get<4>(k), std::get<5>(k), best.split, best.order);
+        std::fprintf(f, "ntt %u %u %u %u %u %u %u r%u\n", std::get<1>(k), std::get<2>(k), std::get<3>(k),
+                     std::get<4>(k), std::get<5>(k), best.split, best.order, REVISION);
         std::fclose(f);
       }
     }
@@ -264,7 +271,9 @@ void tuner_configure(bool enabled, const char* cache_file) {
   if (!f) return;
   char line[256];
   while (std::fgets(line, sizeof line, f)) {
-    unsigned v[8];
+    unsigned v[8], rev;
+    const char* r = std::strchr(line, 'r');
+    if (r && (std::sscanf(r, "r%u", &rev) != 1 || rev != REVISION)) continue;
     if (std::sscanf(line, "ntt %u %u %u %u %u %u %u", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6]) == 7) {
       if (v[5] <= 1 && v[6] <= 1) t.ntt[NKey{dev, v[0], v[1], v[2], v[3], v[4]}] = NttPlan{v[5], v[6]};
       continue;
