@@ -100,9 +100,9 @@ __global__ __launch_bounds__(GKR_THREADS) void k_gkr_eq_pass(uint32_t* buf, cons
 // workgroup's factor (a tree product over lanes), 2^hb lanes the H values'
 // (hb products more), and an entry then costs one product and one 16-byte
 // store. Field products are exact, so the entries equal the pass-by-pass ones.
-// Serial products bind it up to about 2^20 entries: 2^20 took 24 us with
+// Serial products bind it up to about 2^20 entries: 2^20 took 22.2 us with
 // a table of 2^10 low factors built in LDS by ten passes with a barrier each
-// in 64 workgroups, 11 us so (3.3 for the stores alone).
+// in 64 workgroups, 10.6 us so (3.3 for the stores alone).
 constexpr uint32_t GKR_EQ_LO_MAX = 8;  // 2^8 lanes
 constexpr uint32_t GKR_EQ_HB_MAX = 5;
 __device__ __forceinline__ qm31 eq_factor(const uint4* y, uint32_t k, uint32_t i, bool bit) {

@@ -194,7 +194,6 @@ __device__ __forceinline__ void d2_produce(const LeafSrc& L, uint64_t i, G4& g, 
   for (int j = 0; j < 4; j++)
 #pragma unroll
     for (int c = 0; c < 4; c++) acc[j][c] = 0;
-#pragma unroll 2
   for (uint32_t k0 = 0; k0 < K; k0 += 2) {
 #pragma unroll
     for (uint32_t h = 0; h < 2; h++) {

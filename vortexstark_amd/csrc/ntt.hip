@@ -582,8 +582,8 @@ static int radix_shape(const RadixArgs& r) {
 }
 
 template <bool FWD, int MODE, int SHAPE>
-__global__ __launch_bounds__(RX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_radix(uint32_t* dst, const uint32_t* src, RadixArgs a,
-                                                              ColArgs<MODE> cp) {
+__global__ __launch_bounds__(RX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_radix(
+    uint32_t* dst, const uint32_t* src, RadixArgs a, ColArgs<MODE> cp) {
   __shared__ uint32_t lds[1u << RX_E_BITS];
   if constexpr ((MODE & NTT_COLS) != 0) {
     dst = a.cols ? ld_uniform(a.cols + blockIdx.y) : cp.dst[blockIdx.y];
@@ -615,7 +615,8 @@ struct RadixJob {
 };
 
 template <bool FWD, int SHAPE>
-__global__ __launch_bounds__(RX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_radix_list(const RadixJob* jobs, uint32_t n_jobs) {
+__global__ __launch_bounds__(RX_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_radix_list(
+    const RadixJob* jobs, uint32_t n_jobs) {
   __shared__ uint32_t lds[1u << RX_E_BITS];
   const uint64_t b = blockIdx.x;
   uint32_t lo = 0, hi = n_jobs;
