@@ -40,15 +40,26 @@ if int(os.environ.get("GPU_MAX_HW_QUEUES") or 0) < SERVING_HW_QUEUES:
 REFERENCE_MS = 133.0
 # MI355X: 256 CUs x 64 int32 lanes x 2.4 GHz, and with each such instruction a
 # second one of another wavefront, if that is a plain 32-bit add, sub or
-# bitwise operation (half of a compression's are)
-VALU_PEAK_TOPS = 2 * 256 * 64 * 2.4e9 / 1e12
+# bitwise operation (half of a compression's are). So a mix takes at least
+# max(slow operations, all operations / 2) / VALU_ISSUE_TOPS, slow being all
+# but the plain ones.
+VALU_ISSUE_TOPS = 256 * 64 * 2.4e9 / 1e12
+VALU_PEAK_TOPS = 2 * VALU_ISSUE_TOPS
 HBM_PEAK_GBS = 8000.0
 # VALU instructions of one Blake2s compression: 10 rounds x 8 G x
 # (2 add3 + 2 add + 4 xor + 4 rotate)
 OPS_PER_COMPRESSION = 10 * 8 * 12
 # VALU instructions of one canonical M31 butterfly: product (64-bit multiply,
-# fold, conditional subtract: 6), add (3) and subtract (3)
-OPS_PER_BUTTERFLY = 12
+# shift, add, subtract, min), sum (add, subtract, min) and difference
+# (subtract, add, min); the multiply, the shift and the three min are slow
+OPS_PER_BUTTERFLY = 11
+# issue slots, max(slow, all / 2): of a compression (480 of its operations are
+# add3 and rotations), of a butterfly, and of one constraint of the
+# multi-column quotient at one row (eight 64-bit multiply-adds, and the
+# multiply, shift and min of an M31 product)
+SLOTS_PER_COMPRESSION = 480
+SLOTS_PER_BUTTERFLY = 5.5
+SLOTS_PER_CONSTRAINT = 11
 MASK64 = (1 << 64) - 1
 P = 0x7FFFFFFF
 
@@ -207,23 +218,23 @@ VALU_MEASURED_TOPS = 65.0
 # Lane instructions the trace-tree subtree kernel issues per compression
 # (SQ_INSTS_VALU x 64 / compressions, profiles/fib_log24_valu_counters.md):
 # 960 of the compression function plus loads, addressing and stores.
-ISSUED_PER_COMPRESSION = 997.1
+ISSUED_PER_COMPRESSION = 1011.9
 # VALU lane instructions a proof of the serving mix issues on average
 # (rocprofv3 SQ_INSTS_VALU x 64 over `bench.py --profile-serving-mix`, every
-# class of the mix proved eagerly, per-class table setup left out): the
-# issue-rate ceiling of the mix in proofs/s is the VALU rate over it.
-MIX_ISSUED_PER_PROOF = 2.493e10
+# class of the mix proved eagerly, per-class table setup left out,
+# profiles/serving_mix_valu_counters.md). With a second instruction issued
+# along with every one, no schedule gets past VALU_PEAK_TOPS over it.
+MIX_ISSUED_PER_PROOF = 2.395e10
 
 
-def proof_valu_ops(air, log_n, blowup_bits, pow_bits, n_cols=34, n_cons=35):
-    """Algorithmic VALU instructions of one proof: Blake2s compressions of
+def proof_valu_slots(air, log_n, blowup_bits, pow_bits, n_cols=34, n_cons=35):
+    """Algorithmic VALU issue slots of one proof: Blake2s compressions of
     every tree (a leaf of <= 16 words is one compression, a node one) and of
-    the expected PoW search (2^pow_bits nonces), times 960; the NTT
-    butterflies (interpolate on 2^log_n, LDE of log_n layers on 2^le points),
-    times 12; for the multi-column AIR the quotient's 35 constraints at about
-    14 instructions per constraint and row (one M31 product, two QM31 x M31
-    lazy multiply-adds). Folds, decommitment and transcript are left out
-    (under 1 %)."""
+    the expected PoW search (2^pow_bits nonces); the NTT butterflies
+    (interpolate on 2^log_n, LDE of log_n layers on 2^le points); for the
+    multi-column AIR the quotient's 35 constraints at every row (one M31
+    product, two QM31 x M31 lazy multiply-adds each). Folds, decommitment and
+    transcript are left out."""
     n, N = 1 << log_n, 1 << (log_n + blowup_bits)
     le = log_n + blowup_bits
     trees = (2 * N - 1) * (2 if air == 0 else 1 + -(-n_cols // 16))  # trace tree(s) + quotient tree
@@ -231,20 +242,19 @@ def proof_valu_ops(air, log_n, blowup_bits, pow_bits, n_cols=34, n_cons=35):
     comp = trees + fri + ((1 << pow_bits) if pow_bits else 0)
     w = 1 if air == 0 else n_cols
     butterflies = w * log_n * (n // 2 + N // 2)
-    quot = 0 if air == 0 else N * n_cons * 14
-    return comp * OPS_PER_COMPRESSION + butterflies * OPS_PER_BUTTERFLY + quot
+    quot = 0 if air == 0 else N * n_cons * SLOTS_PER_CONSTRAINT
+    return comp * SLOTS_PER_COMPRESSION + butterflies * SLOTS_PER_BUTTERFLY + quot
 
 
 def serving_floor():
-    """The serving mix's VALU floor in proofs/s: the peak VALU rate over the
-    mean algorithmic instructions per proof of the mix (half Fibonacci with
-    log_n uniform in 14..22, half the 34-column AIR with log_n uniform in
-    14..20; blowup 4, PoW 20)."""
-    fib = [proof_valu_ops(0, L, 2, 20) for L in range(14, 23)]
-    d2 = [proof_valu_ops(1, L, 2, 20) for L in range(14, 21)]
+    """The serving mix's VALU floor in proofs/s: the issue rate over the mean
+    algorithmic issue slots per proof of the mix (half Fibonacci with log_n
+    uniform in 14..22, half the 34-column AIR with log_n uniform in 14..20;
+    blowup 4, PoW 20)."""
+    fib = [proof_valu_slots(0, L, 2, 20) for L in range(14, 23)]
+    d2 = [proof_valu_slots(1, L, 2, 20) for L in range(14, 21)]
     mean = 0.5 * sum(fib) / len(fib) + 0.5 * sum(d2) / len(d2)
-    return {"ops_per_proof_mean": round(mean), "floor_proofs_per_s": round(VALU_PEAK_TOPS * 1e12 / mean, 1),
-            "floor_proofs_per_s_measured_rate": round(VALU_MEASURED_TOPS * 1e12 / mean, 1)}
+    return {"issue_slots_per_proof_mean": round(mean), "floor_proofs_per_s": round(VALU_ISSUE_TOPS * 1e12 / mean, 1)}
 
 
 def percentile(xs, q):
@@ -341,13 +351,11 @@ def serving(vx, n_requests, slots, seed=42, load=0.8):
     roof["achieved_proofs_per_s"] = sat_batch["proofs_per_s"]
     roof["frac"] = round(sat_batch["proofs_per_s"] / roof["floor_proofs_per_s"], 4)
     roof["plain_loop_frac"] = round(sat_plain["proofs_per_s"] / roof["floor_proofs_per_s"], 4)
-    ceiling = VALU_MEASURED_TOPS * 1e12 / MIX_ISSUED_PER_PROOF
+    ceiling = VALU_PEAK_TOPS * 1e12 / MIX_ISSUED_PER_PROOF
     roof["issued_instructions_per_proof"] = MIX_ISSUED_PER_PROOF
     roof["issue_ceiling_proofs_per_s"] = round(ceiling, 1)
     roof["frac_of_issue_ceiling"] = round(sat_batch["proofs_per_s"] / ceiling, 4)
     roof["plain_loop_frac_of_issue_ceiling"] = round(sat_plain["proofs_per_s"] / ceiling, 4)
-    # a capacity ratio of 2 needs the batched server at twice the loop
-    roof["ratio_2_needs_frac_of_issue_ceiling"] = round(2 * sat_plain["proofs_per_s"] / ceiling, 4)
     resident = batch.resident_bytes
     plain.close()
     batch.close()
@@ -1185,7 +1193,7 @@ def main():
                          "frac": round(lde_gbs / HBM_PEAK_GBS, 4), "stage_ms": round(stages["lde"], 4),
                          "algorithmic_bytes": lde_bytes,
                          "valu_tops": round(lde_tops, 2), "valu_frac": round(lde_tops / VALU_PEAK_TOPS, 4),
-                         "note": "VALU-bound: 12 int ops per butterfly; the HBM fraction is not the limit"},
+                         "note": "VALU-bound: 11 int ops per butterfly; the HBM fraction is not the limit"},
         "stages_ms": {k: round(v, 4) for k, v in stages.items()},
         "proof_bytes": len(proof),
         "proof_sha256": digest,
