@@ -275,10 +275,7 @@ __global__ void k_write_words(uint32_t* dst, WordWrites w) {
   if (threadIdx.x < w.n) dst[w.at[threadIdx.x]] = w.value[threadIdx.x];
 }
 
-// A few words at scattered places by one launch. (With four or five synchronous
-// copies from pageable memory in its place creating a prover took longer: at
-// log_n = 4 213 us against 188, at 8 338 against 268, at 20 1,265 against
-// 1,218, on one box.)
+// A few words at scattered places by one launch.
 void write_words(uint32_t* dst, const WordWrites& w, hipStream_t s) {
   if (w.n == 0) return;
   hipLaunchKernelGGL(k_write_words, dim3(1), dim3(64), 0, s, dst, w);

@@ -173,6 +173,7 @@ class StarkProver {
   bool timed_ = false;
   bool use_graph_ = true;
   bool tuned_ = false;
+  bool header_written_ = false;
   hipGraphExec_t graph_ = nullptr;
 };
 
