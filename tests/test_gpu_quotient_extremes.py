@@ -1,6 +1,7 @@
 """Numerators and their combination where the kernels' 64-bit sums are largest
 (every value P - 1) and where they vanish, at column counts around the step of
-four and row counts around a workgroup's 2048. Against the oracle."""
+four and row counts around 2048 (one row per lane; test_gpu_combine_rows has
+the counts around workgroups of eight rows per lane). Against the oracle."""
 import numpy as np
 import pytest
 

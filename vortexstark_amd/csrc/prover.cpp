@@ -313,9 +313,7 @@ StarkProver::StarkProver(uint32_t log_n, uint32_t blowup_bits, uint32_t n_querie
 // own, the first on its stream, 50 us more, and with a synchronous copy for each
 // run of words 147 us.)
 void StarkProver::write_header() {
-  if (header_written_) return;
-  header_written_ = true;
-  if (air_.kind == AIR_BATCH) return;
+  if (header_written_ || air_.kind == AIR_BATCH) return;
   WordWrites w{};
   auto put = [&](uint64_t word, std::initializer_list<uint32_t> v) {
     for (uint32_t x : v) w.add((uint32_t)word++, x);
@@ -330,6 +328,7 @@ void StarkProver::write_header() {
   put(layout_.w_nfri, {n_fri_});
   put(layout_.w_nfdec, {n_fri_});
   write_words(proof_.u32(), w, stream_);
+  header_written_ = true;
 }
 
 // Work lists, lifted column table, column offsets and the constant header
